@@ -19,6 +19,10 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+#include <immintrin.h>
+#endif
+
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -406,6 +410,36 @@ int ensure_prefill_capacity(grout_engine* e, int rows) {
   return GROUT_OK;
 }
 
+// f16 logits to f32 on the host.  Compiled for a baseline x86-64 the widening
+// is a library call per value: 385 us for 151936 logits, a fifth of a 4B decode
+// step.  With F16C (every x86-64 server CPU since 2013; checked at run time)
+// eight values convert per instruction, with the same bits.
+void widen_logits_any(const uint16_t* src, float* dst, int n) {
+  for (int i = 0; i < n; ++i) {
+    _Float16 h;
+    std::memcpy(&h, &src[i], 2);
+    dst[i] = (float)h;
+  }
+}
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+__attribute__((target("avx,f16c"))) void widen_logits_f16c(const uint16_t* src, float* dst,
+                                                           int n) {
+  int i = 0;
+  for (; i + 8 <= n; i += 8)
+    _mm256_storeu_ps(dst + i, _mm256_cvtph_ps(_mm_loadu_si128(
+                                  reinterpret_cast<const __m128i*>(src + i))));
+  widen_logits_any(src + i, dst + i, n - i);
+}
+#endif
+
+void widen_logits(const uint16_t* src, float* dst, int n) {
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+  if (__builtin_cpu_supports("avx") && __builtin_cpu_supports("f16c"))
+    return widen_logits_f16c(src, dst, n);
+#endif
+  widen_logits_any(src, dst, n);
+}
+
 int copy_logits_out(grout_engine* e, float* logits_out, uint32_t* next_token) {
   const int V = e->cfg.vocab_size;
   if (logits_out)
@@ -417,13 +451,7 @@ int copy_logits_out(grout_engine* e, float* logits_out, uint32_t* next_token) {
                                           hipMemcpyDeviceToHost, e->stream),
                            "token D2H"));
   GROUT_CHECK(hip_status(hipStreamSynchronize(e->stream), "hipStreamSynchronize"));
-  if (logits_out) {
-    for (int i = 0; i < V; ++i) {
-      _Float16 h;
-      std::memcpy(&h, &e->h_logits[i], 2);
-      logits_out[i] = (float)h;
-    }
-  }
+  if (logits_out) widen_logits(e->h_logits, logits_out, V);
   if (next_token) *next_token = *e->h_token;
   return GROUT_OK;
 }
