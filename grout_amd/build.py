@@ -31,6 +31,7 @@ SOURCES = [
     ("attn_prefill.hip", []),
     ("model_kernels.hip", []),
     ("quant_gemv.hip", []),
+    ("tok_gemm.hip", []),
     ("api.cpp", ["-x", "hip"]),
     ("engine.cpp", ["-x", "hip"]),
     ("loader.cpp", ["-x", "hip"]),

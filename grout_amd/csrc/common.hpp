@@ -71,6 +71,31 @@ inline DivBy make_div(int d) {
   return DivBy{(uint32_t)(((1ull << (31 + l)) + (uint64_t)d - 1) / (uint64_t)d), 31 + l};
 }
 
+// fp32 partial sums of a projection ([splits][rows][ld], tok_gemm.hip) as its
+// consumer reads them: the sum in range order, rounded to f16 once.
+struct Parts {
+  const float* p;  // nullptr: the projection's f16 rows are read instead
+  int splits;
+  long stride;  // floats from one range's sums to the next's
+};
+__device__ __forceinline__ half8 load_parts8(const Parts& a, size_t off) {
+  floatx4 lo = *reinterpret_cast<const floatx4*>(a.p + off);
+  floatx4 hi = *reinterpret_cast<const floatx4*>(a.p + off + 4);
+#pragma unroll 4
+  for (int s = 1; s < a.splits; ++s) {
+    const float* q = a.p + (size_t)s * a.stride + off;
+    lo += *reinterpret_cast<const floatx4*>(q);
+    hi += *reinterpret_cast<const floatx4*>(q + 4);
+  }
+  half8 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    o[e] = (half_t)lo[e];
+    o[4 + e] = (half_t)hi[e];
+  }
+  return o;
+}
+
 // Lane l ends with f(x[l], x[l ^ 16]) and then f(.., x[l ^ 32]): the reduction
 // over the four 16-lane groups that hold one MFMA column, on the VALU
 // (v_permlane16/32_swap, gfx950) instead of two LDS round trips.

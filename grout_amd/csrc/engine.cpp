@@ -93,7 +93,14 @@ struct DecodeBufs {
 // Prefill activations: cap rows.
 struct PrefillBufs {
   size_t ids, hidden, normed, hidden_after_attn, qkv, q_rope, attn_out, attn_proj, ff_normed,
-      gate_up, ff, ff_down;
+      gate_up, ff, ff_down, parts;
+};
+
+// A projection's rows as its consumer reads them: f16 rows, or (splits > 1)
+// fp32 partial sums [splits][rows][columns].
+struct Proj {
+  int splits = 1;
+  const float* parts = nullptr;
 };
 
 __global__ void set_step_kernel(uint32_t* d_token, uint32_t token, uint32_t* d_pos,
@@ -194,13 +201,6 @@ int gemm_rows(grout_engine* e, const void* W, const void* x, void* y, int rows, 
       "rocblas_gemm_ex");
 }
 
-// Projection of `rows` tokens by an f16 matrix.  One row uses the decode
-// GEMV kernel.
-int project(grout_engine* e, const void* W, const void* x, void* y, int rows, int n, int k) {
-  if (rows == 1) return hip_status(grout::launch_gemv(W, x, y, n, k, e->stream), "gemv");
-  return gemm_rows(e, W, x, y, rows, n, k, n);
-}
-
 // One token through one weight part with the decode GEMV of its format.
 int mat_gemv(grout_engine* e, const Mat& m, const void* x, void* y, int k) {
   if (m.fmt == GROUT_WFMT_F16)
@@ -223,13 +223,57 @@ int mat_f16(grout_engine* e, const Mat& m, int k, const void** w) {
   return GROUT_OK;
 }
 
-// Projection of `rows` tokens by one part into columns [0, m.rows) of y
-// (rows ldy apart).
-int mat_project(grout_engine* e, const Mat& m, const void* x, void* y, int rows, int k, int ldy) {
-  if (m.fmt == GROUT_WFMT_F16 && ldy == m.rows) return project(e, m.data, x, y, rows, m.rows, k);
-  const void* w = nullptr;
-  GROUT_CHECK(mat_f16(e, m, k, &w));
-  return gemm_rows(e, w, x, y, rows, m.rows, k, ldy);
+// Projection of `rows` tokens by `np` parts (their rows follow each other)
+// into [rows][n] rows y, n the parts' rows in all.  A few tokens go through
+// the token GEMM, which may leave fp32 partial sums in `parts` instead of f16
+// rows (out says which); one token through the decode GEMVs; more through the
+// library's GEMM, a low-bit matrix after one dequantization.
+int project_rows(grout_engine* e, const Mat* m, int np, const void* x, uint16_t* y, float* parts,
+                 int rows, int k, Proj* out) {
+  int n = 0;
+  bool few = true;
+  for (int i = 0; i < np; ++i) {
+    few = few && grout::tok_gemm_ok(m[i].fmt, rows, m[i].rows, k);
+    n += m[i].rows;
+  }
+  *out = Proj{};
+  if (few) {
+    out->splits = grout::tok_gemm_splits(rows, n, k);
+    out->parts = parts;
+  }
+  int col = 0;
+  for (int i = 0; i < np; ++i) {
+    if (few) {
+      GROUT_CHECK(hip_status(grout::launch_tok_gemm(m[i].fmt, m[i].data, x, y + col, parts + col, n,
+                                                    rows, m[i].rows, k, out->splits, e->stream),
+                             "tok_gemm"));
+    } else if (rows == 1) {
+      GROUT_CHECK(mat_gemv(e, m[i], x, y + col, k));
+    } else {
+      const void* w = nullptr;
+      GROUT_CHECK(mat_f16(e, m[i], k, &w));
+      GROUT_CHECK(gemm_rows(e, w, x, y + col, rows, m[i].rows, k, n));
+    }
+    col += m[i].rows;
+  }
+  return GROUT_OK;
+}
+
+// Bytes of partial sums project_rows may leave for up to `cap` rows.
+size_t parts_bytes(const grout_engine* e, int cap) {
+  const auto& c = e->cfg;
+  size_t mx = 0;
+  auto see = [&](int n, int k) {
+    for (int r = 2; r <= std::min(cap, grout::kTokMax); ++r) {
+      const int s = grout::tok_gemm_splits(r, n, k);
+      if (s > 1) mx = std::max(mx, (size_t)s * r * n * sizeof(float));
+    }
+  };
+  see(e->qkv_dim, c.hidden_size);
+  see(c.hidden_size, e->q_dim);
+  see(2 * c.intermediate_size, c.hidden_size);
+  see(c.hidden_size, c.intermediate_size);
+  return mx;
 }
 
 // Token-embedding rows for ids (device memory).
@@ -251,14 +295,28 @@ int norm(grout_engine* e, const void* residual, const void* x, const void* w, vo
                     "rms_norm");
 }
 
+// add_rms_norm whose x is a projection's rows (row `row0` on).
+int norm_proj(grout_engine* e, const void* residual, const void* x, const Proj& p, size_t row0,
+              const void* w, void* out, void* residual_out, int rows) {
+  const int H = e->cfg.hidden_size;
+  if (p.splits == 1)
+    return norm(e, residual, static_cast<const uint16_t*>(x) + row0 * H, w, out, residual_out,
+                rows);
+  return hip_status(grout::launch_add_rms_norm_parts(
+                        residual, p.parts + row0 * H, p.splits, (long)(row0 + rows) * H, w, out,
+                        residual_out, rows, H, e->cfg.rms_norm_eps, e->stream),
+                    "add_rms_norm");
+}
+
 // Final norm (folding the last layer's residual add), lm_head and argmax
-// over one token's hidden state; leaves f16 logits and the token on device
+// over the hidden state of token `row`; leaves f16 logits and the token on device
 // (and, when advance_pos is set, moves that position word on by one).
-int head(grout_engine* e, const void* hidden_after_attn, const void* ff_down,
-         uint32_t* advance_pos = nullptr) {
+int head(grout_engine* e, const void* hidden_after_attn, const void* ff_down, const Proj& down,
+         size_t row, uint32_t* advance_pos = nullptr) {
   const auto& c = e->cfg;
-  GROUT_CHECK(norm(e, hidden_after_attn, ff_down, e->final_norm, e->d(e->db.normed),
-                   e->d(e->db.hidden), 1));
+  GROUT_CHECK(norm_proj(e, static_cast<const uint16_t*>(hidden_after_attn) + row * c.hidden_size,
+                        ff_down, down, row, e->final_norm, e->d(e->db.normed),
+                        e->d(e->db.hidden), 1));
   GROUT_CHECK(mat_gemv(e, e->lm_head, e->d(e->db.normed), e->d(e->db.logits), c.hidden_size));
   return hip_status(grout::launch_argmax(e->d(e->db.logits), e->d<float>(e->db.argmax_max),
                                          e->d<uint32_t>(e->db.argmax_idx), c.vocab_size,
@@ -330,7 +388,7 @@ int record_decode_step(grout_engine* e) {
   }
   // The step leaves the next step's token (the greedy argmax) and position
   // behind, so a greedy decode loop needs no write of its own per token.
-  return head(e, e->d(b.hidden_after_attn), e->d(b.ff_down), e->d<uint32_t>(b.pos));
+  return head(e, e->d(b.hidden_after_attn), e->d(b.ff_down), Proj{}, 0, e->d<uint32_t>(b.pos));
 }
 
 int capture_decode_graph(grout_engine* e) {
@@ -404,6 +462,7 @@ int ensure_prefill_capacity(grout_engine* e, int rows) {
   b.gate_up = a.take(r * 2 * I * h2);
   b.ff = a.take(r * I * h2);
   b.ff_down = a.take(r * H * h2);
+  b.parts = a.take(parts_bytes(e, cap));
   GROUT_CHECK(hip_status(hipMalloc(&a.base, a.used), "hipMalloc(prefill buffers)"));
   e->pre = a;
   e->prefill_cap = cap;
@@ -1045,53 +1104,56 @@ int run_chunk(grout_engine* e, const uint32_t* tokens, int n, int pos0, float* l
   const int qd = e->q_dim, kd = e->kv_dim;
   const int qkvd = e->qkv_dim;
   uint16_t* const qkv = e->p<uint16_t>(b.qkv);
+  // one buffer of partial sums: each projection's are consumed by the launch
+  // that follows it
+  float* const parts = e->p<float>(b.parts);
+  Proj down;
   for (int l = 0; l < c.num_layers; ++l) {
     const LayerW& w = e->layers[l];
     if (l == 0)
       GROUT_CHECK(norm(e, nullptr, e->p(b.hidden), w.input_norm, e->p(b.normed), nullptr, n));
     else
-      GROUT_CHECK(norm(e, e->p(b.hidden_after_attn), e->p(b.ff_down), w.input_norm,
-                       e->p(b.normed), e->p(b.hidden), n));
-    // one projection per part into its columns of the fused [n][Q|K|V] rows
-    // (one GEMM of 6144 columns measured 26-28 us at 512 tokens against 48 us
-    // for separate Q, K and V GEMMs, Qwen3-4B)
-    int row0 = 0;
-    for (int i = 0; i < w.nqkv; ++i) {
-      const Mat& m = w.qkv[i];
-      const void* wf = nullptr;
-      GROUT_CHECK(mat_f16(e, m, H, &wf));
-      if (n == 1 && m.fmt == GROUT_WFMT_F16)
-        GROUT_CHECK(hip_status(grout::launch_gemv(wf, e->p(b.normed), qkv + row0, m.rows, H, s),
-                               "gemv"));
-      else
-        GROUT_CHECK(gemm_rows(e, wf, e->p(b.normed), qkv + row0, n, m.rows, H, qkvd));
-      row0 += m.rows;
-    }
-    GROUT_CHECK(hip_status(
-        grout::launch_qk_norm_rope_kv_prefill(
-            qkv, qkv + qd, qkv + qd + kd, w.q_norm, w.k_norm, e->rope_cos(), e->rope_sin(),
-            e->p(b.q_rope), e->k_cache(l), e->v_cache(l), pos0, n, c.num_q_heads,
-            c.num_kv_heads, e->head_stride, c.max_ctx, c.rms_norm_eps, s, qkvd, qkvd),
-        "qk_norm_rope_kv_prefill"));
+      GROUT_CHECK(norm_proj(e, e->p(b.hidden_after_attn), e->p(b.ff_down), down, 0, w.input_norm,
+                            e->p(b.normed), e->p(b.hidden), n));
+    // every part writes its columns of the fused [n][Q|K|V] rows (one GEMM of
+    // 6144 columns measured 26-28 us at 512 tokens against 48 us for separate
+    // Q, K and V GEMMs, Qwen3-4B)
+    Proj p;
+    GROUT_CHECK(project_rows(e, w.qkv, w.nqkv, e->p(b.normed), qkv, parts, n, H, &p));
+    if (p.splits == 1)
+      GROUT_CHECK(hip_status(
+          grout::launch_qk_norm_rope_kv_prefill(
+              qkv, qkv + qd, qkv + qd + kd, w.q_norm, w.k_norm, e->rope_cos(), e->rope_sin(),
+              e->p(b.q_rope), e->k_cache(l), e->v_cache(l), pos0, n, c.num_q_heads,
+              c.num_kv_heads, e->head_stride, c.max_ctx, c.rms_norm_eps, s, qkvd, qkvd),
+          "qk_norm_rope_kv_prefill"));
+    else
+      GROUT_CHECK(hip_status(
+          grout::launch_qk_norm_rope_kv_parts(
+              p.parts, p.splits, w.q_norm, w.k_norm, e->rope_cos(), e->rope_sin(), e->p(b.q_rope),
+              e->k_cache(l), e->v_cache(l), pos0, n, c.num_q_heads, c.num_kv_heads,
+              e->head_stride, c.rms_norm_eps, s),
+          "qk_norm_rope_kv_parts"));
     GROUT_CHECK(grout_fmha_prefill(e->p(b.q_rope), e->k_cache(l), e->v_cache(l),
                                    e->p(b.attn_out), n, pos0, c.num_q_heads, c.num_kv_heads, 128,
                                    e->head_stride, e->qk_scale, s));
-    GROUT_CHECK(mat_project(e, w.o, e->p(b.attn_out), e->p(b.attn_proj), n, qd, H));
-    GROUT_CHECK(norm(e, e->p(b.hidden), e->p(b.attn_proj), w.post_norm, e->p(b.ff_normed),
-                     e->p(b.hidden_after_attn), n));
-    row0 = 0;
-    for (int i = 0; i < w.ngu; ++i) {
-      GROUT_CHECK(mat_project(e, w.gu[i], e->p(b.ff_normed), e->p<uint16_t>(b.gate_up) + row0, n,
-                              H, 2 * I));
-      row0 += w.gu[i].rows;
-    }
-    GROUT_CHECK(hip_status(grout::launch_silu_mul(e->p(b.gate_up), e->p(b.ff), n, I, s),
-                           "silu_mul"));
-    GROUT_CHECK(mat_project(e, w.down, e->p(b.ff), e->p(b.ff_down), n, I, H));
+    GROUT_CHECK(project_rows(e, &w.o, 1, e->p(b.attn_out), e->p<uint16_t>(b.attn_proj), parts, n,
+                             qd, &p));
+    GROUT_CHECK(norm_proj(e, e->p(b.hidden), e->p(b.attn_proj), p, 0, w.post_norm,
+                          e->p(b.ff_normed), e->p(b.hidden_after_attn), n));
+    GROUT_CHECK(project_rows(e, w.gu, w.ngu, e->p(b.ff_normed), e->p<uint16_t>(b.gate_up), parts,
+                             n, H, &p));
+    if (p.splits == 1)
+      GROUT_CHECK(hip_status(grout::launch_silu_mul(e->p(b.gate_up), e->p(b.ff), n, I, s),
+                             "silu_mul"));
+    else
+      GROUT_CHECK(hip_status(grout::launch_silu_mul_parts(p.parts, p.splits, e->p(b.ff), n, I, s),
+                             "silu_mul"));
+    GROUT_CHECK(project_rows(e, &w.down, 1, e->p(b.ff), e->p<uint16_t>(b.ff_down), parts, n, I,
+                             &down));
   }
   // Only the last token's logits are needed (src/model.rs api_prefill_logits).
-  const size_t last = (size_t)(n - 1) * H;
-  GROUT_CHECK(head(e, e->p<uint16_t>(b.hidden_after_attn) + last, e->p<uint16_t>(b.ff_down) + last));
+  GROUT_CHECK(head(e, e->p(b.hidden_after_attn), e->p(b.ff_down), down, (size_t)n - 1));
   GROUT_CHECK(copy_logits_out(e, logits_out, next_token));
   e->next_pos = pos0 + n;
   e->session_active = true;

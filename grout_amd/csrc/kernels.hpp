@@ -15,6 +15,13 @@ hipError_t launch_qk_norm_rope_kv_prefill(const void* q, const void* k, const vo
                                           int seq_len, int Hq, int Hkv, long head_stride,
                                           int max_ctx, float eps, hipStream_t stream,
                                           long ldq = 0, long ldkv = 0);
+// The same over the QKV projection's partial sums (splits > 1): rows [Q|K|V]
+// of Hq + 2 Hkv heads, part [splits][seq_len][(Hq + 2 Hkv) * 128].
+hipError_t launch_qk_norm_rope_kv_parts(const float* part, int splits, const void* gamma_q,
+                                        const void* gamma_k, const float* rope_cos,
+                                        const float* rope_sin, void* q_out, void* k_cache,
+                                        void* v_cache, int pos0, int seq_len, int Hq, int Hkv,
+                                        long head_stride, float eps, hipStream_t stream);
 
 hipError_t launch_qk_norm_rope_kv_decode(const void* qkv, const void* gamma_q,
                                          const void* gamma_k, const float* rope_cos,
@@ -66,7 +73,17 @@ hipError_t launch_embedding(const uint32_t* ids, const void* table, void* out, i
                             int vocab, hipStream_t stream);
 hipError_t launch_rms_norm(const void* residual, const void* x, const void* w, void* out,
                            void* residual_out, int rows, int H, float eps, hipStream_t stream);
+// out = norm(residual + x), residual_out = residual + x for x = the rows of a
+// projection's partial sums: part points at the first row, rows H apart,
+// ranges split_stride floats apart.
+hipError_t launch_add_rms_norm_parts(const void* residual, const float* part, int splits,
+                                     long split_stride, const void* w, void* out,
+                                     void* residual_out, int rows, int H, float eps,
+                                     hipStream_t stream);
 hipError_t launch_silu_mul(const void* gate_up, void* out, int rows, int I, hipStream_t stream);
+// The same over partial sums [splits][rows][2 I].
+hipError_t launch_silu_mul_parts(const float* part, int splits, void* out, int rows, int I,
+                                 hipStream_t stream);
 hipError_t launch_gemv(const void* W, const void* x, void* y, int N, int K, hipStream_t stream);
 // GEMV whose input is the RMSNorm (residual == nullptr) or add-RMSNorm of x,
 // computed per wave; the first wave writes residual_out = residual + x.
@@ -104,6 +121,17 @@ hipError_t launch_qgather(int fmt, const void* W, int N, int K, const uint32_t* 
                           void* out, hipStream_t stream);
 hipError_t launch_qweight_dequant(int fmt, const void* W, int N, int K, void* out,
                                   hipStream_t stream);
+
+// Projections of a few tokens (tok_gemm.hip): y[t][n] = x[t] . W[n] for M
+// tokens, x [M][K] f16, W f16 rows (fmt 0) or a repacked low-bit matrix.
+// splits == 1 writes f16 rows ldy apart; more write the fp32 sums of each
+// range of K to part[range][M][ldy].  y / part point at the matrix's first
+// column.
+constexpr int kTokMax = 480;  // no format takes more tokens
+bool tok_gemm_ok(int fmt, int M, int N, int K);
+int tok_gemm_splits(int M, int N, int K);
+hipError_t launch_tok_gemm(int fmt, const void* W, const void* x, void* y, float* part, long ldy,
+                           int M, int N, int K, int splits, hipStream_t stream);
 
 // Writes the 16x16 C fragment of A x B for A[i][k] = i*32+k (k < 32), B = I
 // padded, one float per (lane, element): used to confirm the MFMA lane layout.

@@ -58,10 +58,11 @@ __global__ __launch_bounds__(256) void embedding_kernel(const uint32_t* __restri
 
 // ------------------------------------------------------------- RMSNorm
 
-// One 256-thread workgroup per row; H a multiple of 8.
-template <bool kAdd>
+// One 256-thread workgroup per row; H a multiple of 8.  kParts: x is a
+// projection's partial sums (rows H floats apart).
+template <bool kAdd, bool kParts>
 __global__ __launch_bounds__(256) void rms_norm_kernel(const half_t* __restrict__ residual,
-                                                      const half_t* __restrict__ x,
+                                                      const half_t* __restrict__ x, Parts parts,
                                                       const half_t* __restrict__ w,
                                                       half_t* __restrict__ out,
                                                       half_t* __restrict__ residual_out, int H,
@@ -76,9 +77,11 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const half_t* __restrict_
   for (int it = 0; it < kMaxVec; ++it) {
     const int i = threadIdx.x + it * 256;
     if (i < nvec) {
-      const half8 xv = as_half8(load16(x + row * H + 8 * i));
       half8 rv = {};
       if (kAdd) rv = as_half8(load16(residual + row * H + 8 * i));
+      half8 xv;
+      if constexpr (kParts) xv = load_parts8(parts, row * H + 8 * i);
+      else xv = as_half8(load16(x + row * H + 8 * i));
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         c[it][e] = kAdd ? (float)rv[e] + (float)xv[e] : (float)xv[e];
@@ -110,17 +113,25 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const half_t* __restrict_
 
 // ------------------------------------------------------------- SiLU * up
 
-// gate_up rows are [gate (I) | up (I)]; out rows are I wide.
+// gate_up rows are [gate (I) | up (I)]; out rows are I wide.  kParts: the
+// projection's partial sums instead of its f16 rows.
+template <bool kParts>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const half_t* __restrict__ gate_up,
-                                                      half_t* __restrict__ out, int I,
+                                                      Parts parts, half_t* __restrict__ out, int I,
                                                       long total_vec) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= total_vec) return;
   const int nvec = I / 8;
   const long row = i / nvec;
   const int v = (int)(i - row * nvec);
-  const half8 g = as_half8(load16(gate_up + row * 2 * I + 8 * v));
-  const half8 u = as_half8(load16(gate_up + row * 2 * I + I + 8 * v));
+  half8 g, u;
+  if constexpr (kParts) {
+    g = load_parts8(parts, row * 2 * I + 8 * v);
+    u = load_parts8(parts, row * 2 * I + I + 8 * v);
+  } else {
+    g = as_half8(load16(gate_up + row * 2 * I + 8 * v));
+    u = as_half8(load16(gate_up + row * 2 * I + I + 8 * v));
+  }
   half8 o;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -681,21 +692,43 @@ hipError_t launch_embedding(const uint32_t* ids, const void* table, void* out, i
 hipError_t launch_rms_norm(const void* residual, const void* x, const void* w, void* out,
                            void* residual_out, int rows, int H, float eps, hipStream_t stream) {
   if (H % 8 != 0 || H > 8192) return hipErrorInvalidValue;
+  const Parts none{nullptr, 0, 0};
   if (residual)
-    rms_norm_kernel<true><<<rows, 256, 0, stream>>>((const half_t*)residual, (const half_t*)x,
-                                                    (const half_t*)w, (half_t*)out,
-                                                    (half_t*)residual_out, H, eps);
+    rms_norm_kernel<true, false><<<rows, 256, 0, stream>>>(
+        (const half_t*)residual, (const half_t*)x, none, (const half_t*)w, (half_t*)out,
+        (half_t*)residual_out, H, eps);
   else
-    rms_norm_kernel<false><<<rows, 256, 0, stream>>>(nullptr, (const half_t*)x, (const half_t*)w,
-                                                     (half_t*)out, nullptr, H, eps);
+    rms_norm_kernel<false, false><<<rows, 256, 0, stream>>>(
+        nullptr, (const half_t*)x, none, (const half_t*)w, (half_t*)out, nullptr, H, eps);
+  return hipGetLastError();
+}
+
+hipError_t launch_add_rms_norm_parts(const void* residual, const float* part, int splits,
+                                     long split_stride, const void* w, void* out,
+                                     void* residual_out, int rows, int H, float eps,
+                                     hipStream_t stream) {
+  if (H % 8 != 0 || H > 8192 || residual == nullptr || part == nullptr || splits < 1)
+    return hipErrorInvalidValue;
+  rms_norm_kernel<true, true><<<rows, 256, 0, stream>>>(
+      (const half_t*)residual, nullptr, Parts{part, splits, split_stride}, (const half_t*)w,
+      (half_t*)out, (half_t*)residual_out, H, eps);
   return hipGetLastError();
 }
 
 hipError_t launch_silu_mul(const void* gate_up, void* out, int rows, int I, hipStream_t stream) {
   if (I % 8 != 0) return hipErrorInvalidValue;
   const long total = (long)rows * (I / 8);
-  silu_mul_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>((const half_t*)gate_up,
-                                                                      (half_t*)out, I, total);
+  silu_mul_kernel<false><<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(
+      (const half_t*)gate_up, Parts{nullptr, 0, 0}, (half_t*)out, I, total);
+  return hipGetLastError();
+}
+
+hipError_t launch_silu_mul_parts(const float* part, int splits, void* out, int rows, int I,
+                                 hipStream_t stream) {
+  if (I % 8 != 0 || part == nullptr || splits < 1) return hipErrorInvalidValue;
+  const long total = (long)rows * (I / 8);
+  silu_mul_kernel<true><<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(
+      nullptr, Parts{part, splits, (long)rows * 2 * I}, (half_t*)out, I, total);
   return hipGetLastError();
 }
 

@@ -105,8 +105,12 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_kernel(
 // q_out; K rows to the cache slot, with their V row copied alongside.  The
 // per-row work (the reduction, the fp64 Newton sequence of 1/sqrt) runs once
 // per 8 rows of a wave instead of once per 2 with 32 lanes per row.
+// kParts: the rows come as the QKV projection's partial sums (token rows
+// [Q|K|V]), rounded to f16 here.
+template <bool kParts>
 __global__ __launch_bounds__(256) void qk_norm_rope_kv_prefill8_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
+    Parts parts,
     const half_t* __restrict__ gamma_q, const half_t* __restrict__ gamma_k,
     const float* __restrict__ rope_cos, const float* __restrict__ rope_sin,
     half_t* __restrict__ q_out, half_t* __restrict__ k_cache, half_t* __restrict__ v_cache,
@@ -123,7 +127,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_prefill8_kernel(
   // token s's rows start ldq (q) / ldkv (k, v) elements apart
   const half_t* x = is_q ? q + (size_t)s * ldq + (size_t)h * kHeadDim
                          : k + (size_t)s * ldkv + (size_t)kvh * kHeadDim;
-  const u32x4 xlo = load16(x + 8 * i), xhi = load16(x + 64 + 8 * i);
+  const size_t prow = ((size_t)s * (Hq + 2 * Hkv) + h) * kHeadDim + 8 * i;  // K follows Q
+  const u32x4 xlo = kParts ? as_u32x4(load_parts8(parts, prow)) : load16(x + 8 * i);
+  const u32x4 xhi = kParts ? as_u32x4(load_parts8(parts, prow + 64)) : load16(x + 64 + 8 * i);
   const half_t* gm = is_q ? gamma_q : gamma_k;
   const half8 glo = as_half8(load16(gm + 8 * i)), ghi = as_half8(load16(gm + 64 + 8 * i));
   const float* crow = rope_cos + (size_t)pos * (kHeadDim / 2) + 8 * i;
@@ -134,9 +140,15 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_prefill8_kernel(
   const floatx4 s1 = *reinterpret_cast<const floatx4*>(srow + 4);
   u32x4 vlo = {0u, 0u, 0u, 0u}, vhi = {0u, 0u, 0u, 0u};
   if (!is_q) {
-    const half_t* vr = v + (size_t)s * ldkv + (size_t)kvh * kHeadDim;
-    vlo = load16(vr + 8 * i);
-    vhi = load16(vr + 64 + 8 * i);
+    if constexpr (kParts) {
+      const size_t vrow = prow + (size_t)Hkv * kHeadDim;
+      vlo = as_u32x4(load_parts8(parts, vrow));
+      vhi = as_u32x4(load_parts8(parts, vrow + 64));
+    } else {
+      const half_t* vr = v + (size_t)s * ldkv + (size_t)kvh * kHeadDim;
+      vlo = load16(vr + 8 * i);
+      vhi = load16(vr + 64 + 8 * i);
+    }
   }
   const float c[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
   const float sn[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
@@ -171,10 +183,26 @@ hipError_t launch_qk_norm_rope_kv_prefill(const void* q, const void* k, const vo
     return hipErrorInvalidValue;
   // 32 rows per 256-thread workgroup measured fastest on MI355X (S=2048, 4B:
   // 8.6-8.7 us; 64/128/512 threads 8.9-9.5 us; two rows per lane group 9.8-10.9 us)
-  qk_norm_rope_kv_prefill8_kernel<<<(unsigned)((rows + 31) / 32), 256, 0, stream>>>(
-      (const half_t*)q, (const half_t*)k, (const half_t*)v, (const half_t*)gamma_q,
-      (const half_t*)gamma_k, rope_cos, rope_sin, (half_t*)q_out, (half_t*)k_cache,
-      (half_t*)v_cache, pos0, (int)rows, Hq, Hkv, head_stride, eps, ldq, ldkv);
+  qk_norm_rope_kv_prefill8_kernel<false><<<(unsigned)((rows + 31) / 32), 256, 0, stream>>>(
+      (const half_t*)q, (const half_t*)k, (const half_t*)v, Parts{nullptr, 0, 0},
+      (const half_t*)gamma_q, (const half_t*)gamma_k, rope_cos, rope_sin, (half_t*)q_out,
+      (half_t*)k_cache, (half_t*)v_cache, pos0, (int)rows, Hq, Hkv, head_stride, eps, ldq, ldkv);
+  return hipGetLastError();
+}
+
+hipError_t launch_qk_norm_rope_kv_parts(const float* part, int splits, const void* gamma_q,
+                                        const void* gamma_k, const float* rope_cos,
+                                        const float* rope_sin, void* q_out, void* k_cache,
+                                        void* v_cache, int pos0, int seq_len, int Hq, int Hkv,
+                                        long head_stride, float eps, hipStream_t stream) {
+  const long rows = (long)seq_len * (Hq + Hkv);
+  if (rows <= 0 || rows > 0x7fffffffL || part == nullptr || splits < 1)
+    return hipErrorInvalidValue;
+  const Parts parts{part, splits, (long)seq_len * (Hq + 2 * Hkv) * kHeadDim};
+  qk_norm_rope_kv_prefill8_kernel<true><<<(unsigned)((rows + 31) / 32), 256, 0, stream>>>(
+      nullptr, nullptr, nullptr, parts, (const half_t*)gamma_q, (const half_t*)gamma_k, rope_cos,
+      rope_sin, (half_t*)q_out, (half_t*)k_cache, (half_t*)v_cache, pos0, (int)rows, Hq, Hkv,
+      head_stride, eps, 0, 0);
   return hipGetLastError();
 }
 

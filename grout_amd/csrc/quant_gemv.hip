@@ -25,6 +25,7 @@
 // run's scale (and min) is applied once: scale * sum(q x) - min * sum(x).
 #include "common.hpp"
 #include "kernels.hpp"
+#include "quant_layout.hpp"
 
 #include <atomic>
 
@@ -35,38 +36,6 @@ constexpr int kQMaxK = 32768;  // x staged in LDS (at most 64 KiB): every Qwen3 
                                // <= 107 KiB of LDS (gfx950: 160 KiB per workgroup)
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
-__host__ __device__ inline size_t qalign(size_t b) { return (b + 255) / 256 * 256; }
-
-// Byte offsets of the repacked arrays of an [n][k] matrix and its total size.
-struct QLayout {
-  size_t off[4];
-  size_t total;
-};
-__host__ __device__ inline QLayout qlayout(int fmt, size_t n, size_t k) {
-  QLayout L{};
-  size_t sz[4] = {0, 0, 0, 0};
-  if (fmt == 8) {
-    sz[0] = n * k;
-    sz[1] = n * (k / 32) * 2;
-  } else if (fmt == 12 || fmt == 13) {
-    sz[0] = n * k / 2;
-    sz[1] = n * (k / 256) * 16;
-    if (fmt == 13) sz[2] = n * k / 8;
-  } else if (fmt == 14) {
-    sz[0] = n * k / 2;
-    sz[1] = n * k / 4;
-    sz[2] = n * k / 16;
-    sz[3] = n * (k / 256) * 2;
-  }
-  size_t o = 0;
-  for (int i = 0; i < 4; ++i) {
-    L.off[i] = o;
-    o += qalign(sz[i]);
-  }
-  L.total = o;
-  return L;
-}
 
 // ---------------------------------------------------------------- repack
 
