@@ -98,19 +98,50 @@ int grout_qk_norm_rope_kv_decode(const void* qkv, const void* gamma_q, const voi
                     "qk_norm_rope_kv_decode launch");
 }
 
-int grout_fmha_prefill(const void* q, const void* k_cache, const void* v_cache, void* out,
-                       int seq_len, int pos0, int num_q_heads, int num_kv_heads, int head_dim,
-                       long kv_head_stride, float qk_scale, void* stream) {
+static int check_fmha_prefill(const void* q, const void* k_cache, const void* v_cache,
+                              const void* out, int seq_len, int pos0, int num_q_heads,
+                              int num_kv_heads, int head_dim, long kv_head_stride,
+                              float qk_scale) {
   GROUT_CHECK(check_heads(num_q_heads, num_kv_heads, head_dim, 1 << 20));
   GROUT_NEED(seq_len >= 1, GROUT_EINVAL, "attention requires q_len >= 1");
   GROUT_NEED(pos0 >= 0, GROUT_EINVAL, "pos0=%d", pos0);
   GROUT_NEED(std::isfinite(qk_scale) && qk_scale > 0.f, GROUT_EINVAL, "qk_scale=%g",
              (double)qk_scale);
   GROUT_CHECK(check_ptrs16({{q, "q"}, {k_cache, "k_cache"}, {v_cache, "v_cache"}, {out, "out"}}));
-  GROUT_CHECK(check_stride(kv_head_stride, (long)pos0 + seq_len));
+  return check_stride(kv_head_stride, (long)pos0 + seq_len);
+}
+
+int grout_fmha_prefill(const void* q, const void* k_cache, const void* v_cache, void* out,
+                       int seq_len, int pos0, int num_q_heads, int num_kv_heads, int head_dim,
+                       long kv_head_stride, float qk_scale, void* stream) {
+  GROUT_CHECK(check_fmha_prefill(q, k_cache, v_cache, out, seq_len, pos0, num_q_heads,
+                                 num_kv_heads, head_dim, kv_head_stride, qk_scale));
   return hip_status(grout::launch_fmha_prefill(q, k_cache, v_cache, out, seq_len, pos0,
                                                num_q_heads, num_kv_heads, kv_head_stride,
                                                qk_scale, as_stream(stream)),
+                    "fmha_prefill launch");
+}
+
+size_t grout_fmha_prefill_workspace_bytes(int seq_len, int pos0, int num_q_heads,
+                                          int num_kv_heads) {
+  if (seq_len < 1 || pos0 < 0 || (long)pos0 + seq_len > GROUT_MAX_CTX) return 0;
+  if (check_heads(num_q_heads, num_kv_heads, 128, 1 << 20) != GROUT_OK) return 0;
+  return grout::fmha_prefill_split_bytes(
+      seq_len, num_q_heads,
+      grout::fmha_prefill_splits(seq_len, pos0, num_q_heads, num_kv_heads));
+}
+
+int grout_fmha_prefill_ws(const void* q, const void* k_cache, const void* v_cache, void* out,
+                          void* workspace, size_t workspace_bytes, int seq_len, int pos0,
+                          int num_q_heads, int num_kv_heads, int head_dim, long kv_head_stride,
+                          float qk_scale, void* stream) {
+  GROUT_CHECK(check_fmha_prefill(q, k_cache, v_cache, out, seq_len, pos0, num_q_heads,
+                                 num_kv_heads, head_dim, kv_head_stride, qk_scale));
+  if (workspace) GROUT_CHECK(check_ptrs16({{workspace, "workspace"}}));
+  return hip_status(grout::launch_fmha_prefill(q, k_cache, v_cache, out, seq_len, pos0,
+                                               num_q_heads, num_kv_heads, kv_head_stride,
+                                               qk_scale, as_stream(stream), workspace,
+                                               workspace ? workspace_bytes : 0),
                     "fmha_prefill launch");
 }
 

@@ -60,6 +60,8 @@
 namespace grout {
 
 constexpr int kBN = 64;  // kv positions per tile
+constexpr int kMaxPrefillSplits = 16;  // kv ranges of the split form
+constexpr int kMinSplitTiles = 24;     // tiles up to which one range is kept
 // A lane's share of a tile row sum at or above this, 2^(8 + kPHeadroom),
 // sends the tile down the exact-max path of the speculative softmax (see
 // s_phase).
@@ -117,13 +119,22 @@ struct BlockMap {
   DivBy hkv, nsub;
 };
 
+// Split form: a q block's kv tiles in nsplit ranges, each a workgroup of its
+// own that writes fp32 partials (unnormalized acc [nsplit][S][Hq][128], then
+// (m, l) [nsplit][S][Hq][2]) for fmha_prefill_merge_kernel.
+struct KvSplit {
+  int nsplit;
+  float* acc;
+  float* ml;
+};
+
 // MB: 16-row MFMA blocks per wave (2: 32 rows per wave, 128 per team; 1: 16
 // and 64, for short prompts, where the 128-row form leaves CUs idle).
-template <int HG, int MB>
+template <int HG, int MB, bool SPLIT>
 __global__ __launch_bounds__(512, 1) void fmha_prefill_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k_cache,
     const half_t* __restrict__ v_cache, half_t* __restrict__ out, int S, int pos0, int Hq,
-    int Hkv, long head_stride, float scale_log2, int nqb, int paired, BlockMap bm) {
+    int Hkv, long head_stride, float scale_log2, int nqb, int paired, BlockMap bm, KvSplit ks) {
   constexpr int RT = 64 * MB;  // rows per team
   constexpr int BQ = RT / HG;
   // Per team: two K slots and two V slots, each slot its own LDS object, so
@@ -139,8 +150,10 @@ __global__ __launch_bounds__(512, 1) void fmha_prefill_kernel(
   const int bid = blockIdx.x;
   const int rest = (int)div_by((uint32_t)bid, bm.hkv);
   const int kvh = bid - rest * Hkv;
-  const int r = (int)div_by((uint32_t)rest, bm.nsub);
-  const int hsub = rest - r * nsub;
+  const int rr = (int)div_by((uint32_t)rest, bm.nsub);
+  const int hsub = rest - rr * nsub;
+  const int split = SPLIT ? rr / nqb : 0;
+  const int r = SPLIT ? rr - split * nqb : rr;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -159,7 +172,15 @@ __global__ __launch_bounds__(512, 1) void fmha_prefill_kernel(
   // both forms; unpaired, l = h means no light block.
   const int h = nqb - 1 - r;
   const int l = paired ? r : h;
-  const int th = tiles_of(h), tl = h != l ? tiles_of(l) : 0;
+  // split form: th counts the tiles of this range of block h, from tile base
+  // on (none at all for a range past the block's last tile)
+  int base = 0, th = tiles_of(h);
+  if constexpr (SPLIT) {
+    const int per = (th + ks.nsplit - 1) / ks.nsplit;
+    base = min(split * per, th);
+    th = min(per, th - base);
+  }
+  const int tl = h != l ? tiles_of(l) : 0;
   const int a = (th + tl + 1) / 2;
   const int nB = tl + th - a;
   const bool merge_h = th > a;
@@ -167,11 +188,11 @@ __global__ __launch_bounds__(512, 1) void fmha_prefill_kernel(
   // tiles of q block qb1 from tile tb1 (wave-uniform).
   int qb0, tb0, n0, qb1, tb1, n1;
   if (team == 0) {
-    qb0 = h; tb0 = 0; n0 = a; qb1 = h; tb1 = 0; n1 = 0;
+    qb0 = h; tb0 = base; n0 = a; qb1 = h; tb1 = 0; n1 = 0;
   } else if (tl > 0) {
     qb0 = l; tb0 = 0; n0 = tl; qb1 = h; tb1 = a; n1 = th - a;
   } else {
-    qb0 = h; tb0 = a; n0 = th - a; qb1 = h; tb1 = 0; n1 = 0;
+    qb0 = h; tb0 = base + a; n0 = th - a; qb1 = h; tb1 = 0; n1 = 0;
   }
   const int n = n0 + n1;
   auto tile_at = [&](int j) __attribute__((always_inline)) { return j < n0 ? tb0 + j : tb1 + (j - n0); };
@@ -473,8 +494,19 @@ __global__ __launch_bounds__(512, 1) void fmha_prefill_kernel(
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
       if (!row_valid(qb, mb)) continue;
+      const size_t row = (size_t)(qb * BQ + rpos(mb)) * Hq + rhead(mb);
+      if constexpr (SPLIT) {
+        const size_t prow = (size_t)split * S * Hq + row;
+        float* arow = ks.acc + prow * kHeadDim;
+#pragma unroll
+        for (int db = DB0; db < DB0 + NDB; ++db)
+          *reinterpret_cast<floatx4*>(arow + 16 * db + 4 * kb) = acc[mb][db];
+        if (DB0 == 0 && kb == 0)
+          *reinterpret_cast<float2*>(ks.ml + 2 * prow) = make_float2(m[mb], lrow[mb]);
+        continue;
+      }
       const float inv = 1.0f / lrow[mb];
-      half_t* orow = out + ((size_t)(qb * BQ + rpos(mb)) * Hq + rhead(mb)) * kHeadDim;
+      half_t* orow = out + row * kHeadDim;
 #pragma unroll
       for (int db = DB0; db < DB0 + NDB; ++db) {
         half4 o;
@@ -564,7 +596,7 @@ __global__ __launch_bounds__(512, 1) void fmha_prefill_kernel(
   float lrow[MB];
   row_sums(lrow);
   if (!merge_h) {
-    if (n > 0) write_rows(c0, c8, n1 > 0 ? qb1 : qb0, lrow);
+    if (n > 0 || (SPLIT && team == 0)) write_rows(c0, c8, n1 > 0 ? qb1 : qb0, lrow);
     return;
   }
   // Team B holds tiles [a, T_h) of block h, team A tiles [0, a): same wave
@@ -603,6 +635,7 @@ __global__ __launch_bounds__(512, 1) void fmha_prefill_kernel(
       const float sa = fast_exp2(ma - mn), sb = fast_exp2(mbb - mn);
       const float ss = team == 0 ? sa : sb, so = team == 0 ? sb : sa;
       lrow[mb] = la * sa + lb * sb;
+      if constexpr (SPLIT) m[mb] = mn;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const floatx4 mine = acc[mb][KEEP + i] * ss;
@@ -617,6 +650,36 @@ __global__ __launch_bounds__(512, 1) void fmha_prefill_kernel(
     finish(c0);
   else
     finish(c4);
+}
+
+// Merge of the split form's partials: one query row (position, head) per 32
+// lanes, 4 d per lane; the ranges' (m, l) first, so every load of the row's
+// accumulators is independent.  A range without an unmasked position has
+// m = -1e30, l = 0, acc = 0 and weighs nothing.
+__global__ __launch_bounds__(256) void fmha_prefill_merge_kernel(const float* __restrict__ acc,
+                                                                const float* __restrict__ ml,
+                                                                half_t* __restrict__ out,
+                                                                int rows, int nsplit) {
+  const int row = (int)blockIdx.x * 8 + (int)(threadIdx.x >> 5);
+  if (row >= rows) return;
+  const int d = 4 * (threadIdx.x & 31);
+  float M = -1.0e30f;
+  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, ml[2 * ((size_t)s * rows + row)]);
+  float L = 0.f;
+  floatx4 O = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < nsplit; ++s) {
+    const size_t r = (size_t)s * rows + row;
+    const float2 v = *reinterpret_cast<const float2*>(ml + 2 * r);
+    const float wgt = fast_exp2(v.x - M);
+    L += wgt * v.y;
+    O += wgt * *reinterpret_cast<const floatx4*>(acc + r * kHeadDim + d);
+  }
+  const float inv = 1.0f / L;
+  half4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = (half_t)(O[i] * inv);
+  *reinterpret_cast<u32x2*>(out + (size_t)row * kHeadDim + d) = __builtin_bit_cast(u32x2, o);
 }
 
 // Shared-stream variant: a segment is one 256-row q block, team A holding its
@@ -1042,12 +1105,56 @@ PrefillPlan plan_fmha_prefill(int seq_len, int Hq, int Hkv) {
   return p;
 }
 
+// GROUT_FMHA_PREFILL_SPLITS=n forces n kv ranges (capped at one per tile) in
+// the 64-row single-block form; 1 turns the split off.
+int fmha_prefill_splits(int seq_len, int pos0, int Hq, int Hkv) {
+  const PrefillPlan p = plan_fmha_prefill(seq_len, Hq, Hkv);
+  if (p.shared || p.paired || p.wave_rows != 16) return 1;
+  const int tiles = (int)(((long)pos0 + seq_len + kBN - 1) / kBN);
+  if (const int o = env_override("GROUT_FMHA_PREFILL_SPLITS"); o >= 1)
+    return o < tiles ? (o < kMaxPrefillSplits ? o : kMaxPrefillSplits) : tiles;
+  if (tiles <= kMinSplitTiles) return 1;
+  // A chunk of few rows on a long cache: its q blocks leave CUs idle while each
+  // walks every tile (61 rows at 8131, Qwen3-4B: 32 workgroups of 128 tiles).
+  // Estimated time of n ranges, in units of one tile of one team (~1.1 us):
+  // rounds of 256 workgroups, each ~5 units of prologue and end plus its
+  // tiles over the two teams, and for n > 1 the merge launch (~2.5 units) and
+  // the partials' traffic (0.01 units per workgroup).  Swept over 1-500 rows,
+  // 1k-32k positions, 16-64 heads: the pick is the fastest count or within 10%
+  // of it.  Measured (us, unsplit -> split): 4B heads 61 rows at 8131 70.6 ->
+  // 21.3, at 32000 261 -> 50; 1 row at 8000 69 -> 18; 18 at 32000 260 -> 33;
+  // 256 at 8000 71 -> 50; 32B heads 61 at 8131 70 -> 31.  Up to 24 tiles one
+  // range is as fast (61 rows at 1000: 14.9, split 17).
+  long best = 0;
+  int ns = 1;
+  for (int n = 1; n <= kMaxPrefillSplits && n <= tiles / 4 + 1; ++n) {
+    const long wgs = p.workgroups * n, rounds = (wgs + 255) / 256;
+    const long per = (tiles + n - 1) / n;
+    const long t = 100 * rounds * (5 + (per + 1) / 2) + (n > 1 ? 250 + wgs : 0);
+    if (n == 1 || t < best) {
+      best = t;
+      ns = n;
+    }
+  }
+  return ns;
+}
+
+size_t fmha_prefill_split_bytes(int seq_len, int Hq, int nsplit) {
+  return nsplit < 2 ? 0 : (size_t)nsplit * seq_len * Hq * (kHeadDim + 2) * sizeof(float);
+}
+
 hipError_t launch_fmha_prefill(const void* q, const void* k_cache, const void* v_cache,
                                void* out, int seq_len, int pos0, int Hq, int Hkv,
-                               long head_stride, float qk_scale, hipStream_t stream) {
+                               long head_stride, float qk_scale, hipStream_t stream,
+                               void* workspace, size_t workspace_bytes) {
   const float scale_log2 = qk_scale * 1.4426950408889634f;
   const PrefillPlan p = plan_fmha_prefill(seq_len, Hq, Hkv);
-  const long blocks = p.workgroups;
+  int nsplit = workspace ? fmha_prefill_splits(seq_len, pos0, Hq, Hkv) : 1;
+  while (fmha_prefill_split_bytes(seq_len, Hq, nsplit) > workspace_bytes) --nsplit;
+  const long blocks = p.workgroups * nsplit;
+  const long rows = (long)seq_len * Hq;
+  float* const ws = static_cast<float*>(workspace);
+  const KvSplit ks{nsplit, ws, ws ? ws + (size_t)nsplit * rows * kHeadDim : nullptr};
   const int shared = p.shared, wave_rows = p.wave_rows, paired = p.paired, nqbr = p.nqb,
             nqb2 = p.nqb2;
   if (blocks <= 0 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
@@ -1059,13 +1166,17 @@ hipError_t launch_fmha_prefill(const void* q, const void* k_cache, const void* v
           (const half_t*)q, (const half_t*)k_cache, (const half_t*)v_cache, (half_t*)out,  \
           seq_len, pos0, Hq, Hkv, head_stride, scale_log2, nqb2, paired);                  \
     else if (wave_rows == 32)                                                              \
-      fmha_prefill_kernel<hg, 2><<<(unsigned)blocks, 512, 0, stream>>>(                    \
+      fmha_prefill_kernel<hg, 2, false><<<(unsigned)blocks, 512, 0, stream>>>(             \
           (const half_t*)q, (const half_t*)k_cache, (const half_t*)v_cache, (half_t*)out,  \
-          seq_len, pos0, Hq, Hkv, head_stride, scale_log2, nqbr, paired, bm);                  \
+          seq_len, pos0, Hq, Hkv, head_stride, scale_log2, nqbr, paired, bm, ks);          \
+    else if (nsplit == 1)                                                                  \
+      fmha_prefill_kernel<hg, 1, false><<<(unsigned)blocks, 512, 0, stream>>>(             \
+          (const half_t*)q, (const half_t*)k_cache, (const half_t*)v_cache, (half_t*)out,  \
+          seq_len, pos0, Hq, Hkv, head_stride, scale_log2, nqbr, paired, bm, ks);          \
     else                                                                                   \
-      fmha_prefill_kernel<hg, 1><<<(unsigned)blocks, 512, 0, stream>>>(                    \
+      fmha_prefill_kernel<hg, 1, true><<<(unsigned)blocks, 512, 0, stream>>>(              \
           (const half_t*)q, (const half_t*)k_cache, (const half_t*)v_cache, (half_t*)out,  \
-          seq_len, pos0, Hq, Hkv, head_stride, scale_log2, nqbr, paired, bm);                  \
+          seq_len, pos0, Hq, Hkv, head_stride, scale_log2, nqbr, paired, bm, ks);          \
     break;
   switch (p.HG) {
     GROUT_PREFILL_CASE(1)
@@ -1080,6 +1191,10 @@ hipError_t launch_fmha_prefill(const void* q, const void* k_cache, const void* v
       return hipErrorInvalidValue;
   }
 #undef GROUT_PREFILL_CASE
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess || nsplit == 1) return err;
+  fmha_prefill_merge_kernel<<<(unsigned)((rows + 7) / 8), 256, 0, stream>>>(
+      ks.acc, ks.ml, (half_t*)out, (int)rows, nsplit);
   return hipGetLastError();
 }
 

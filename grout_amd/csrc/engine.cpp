@@ -93,7 +93,7 @@ struct DecodeBufs {
 // Prefill activations: cap rows.
 struct PrefillBufs {
   size_t ids, hidden, normed, hidden_after_attn, qkv, q_rope, attn_out, attn_proj, ff_normed,
-      gate_up, ff, ff_down, parts;
+      gate_up, ff, ff_down, parts, attn_ws;
 };
 
 // A projection's rows as its consumer reads them: f16 rows, or (splits > 1)
@@ -141,6 +141,7 @@ struct grout_engine {
   DecodeBufs db{};
   Arena pre;
   PrefillBufs pb{};
+  size_t attn_ws_bytes = 0;
   int prefill_cap = 0;
   // f16 copy of one low-bit matrix at a time for the prefill GEMMs
   void* deq = nullptr;
@@ -463,6 +464,14 @@ int ensure_prefill_capacity(grout_engine* e, int rows) {
   b.ff = a.take(r * I * h2);
   b.ff_down = a.take(r * H * h2);
   b.parts = a.take(parts_bytes(e, cap));
+  // partials of a chunk's attention at the longest context (a chunk that would
+  // take more gets fewer kv ranges)
+  e->attn_ws_bytes = 0;
+  for (int n = 1; n <= cap; n += n < 64 ? 1 : 16)
+    e->attn_ws_bytes = std::max(
+        e->attn_ws_bytes, grout_fmha_prefill_workspace_bytes(n, c.max_ctx - n, c.num_q_heads,
+                                                             c.num_kv_heads));
+  b.attn_ws = a.take(e->attn_ws_bytes);
   GROUT_CHECK(hip_status(hipMalloc(&a.base, a.used), "hipMalloc(prefill buffers)"));
   e->pre = a;
   e->prefill_cap = cap;
@@ -1134,9 +1143,10 @@ int run_chunk(grout_engine* e, const uint32_t* tokens, int n, int pos0, float* l
               e->k_cache(l), e->v_cache(l), pos0, n, c.num_q_heads, c.num_kv_heads,
               e->head_stride, c.rms_norm_eps, s),
           "qk_norm_rope_kv_parts"));
-    GROUT_CHECK(grout_fmha_prefill(e->p(b.q_rope), e->k_cache(l), e->v_cache(l),
-                                   e->p(b.attn_out), n, pos0, c.num_q_heads, c.num_kv_heads, 128,
-                                   e->head_stride, e->qk_scale, s));
+    GROUT_CHECK(grout_fmha_prefill_ws(e->p(b.q_rope), e->k_cache(l), e->v_cache(l),
+                                      e->p(b.attn_out), e->p(b.attn_ws), e->attn_ws_bytes, n, pos0,
+                                      c.num_q_heads, c.num_kv_heads, 128, e->head_stride,
+                                      e->qk_scale, s));
     GROUT_CHECK(project_rows(e, &w.o, 1, e->p(b.attn_out), e->p<uint16_t>(b.attn_proj), parts, n,
                              qd, &p));
     GROUT_CHECK(norm_proj(e, e->p(b.hidden), e->p(b.attn_proj), p, 0, w.post_norm,

@@ -63,9 +63,16 @@ struct PrefillPlan {
   long workgroups = 0;
 };
 PrefillPlan plan_fmha_prefill(int seq_len, int Hq, int Hkv);
+// kv ranges the 64-row single-block form takes for a chunk at pos0 (1: none),
+// and the bytes of its fp32 partials.
+int fmha_prefill_splits(int seq_len, int pos0, int Hq, int Hkv);
+size_t fmha_prefill_split_bytes(int seq_len, int Hq, int nsplit);
+// workspace: fmha_prefill_split_bytes of fmha_prefill_splits; as many ranges as
+// a smaller one holds are used, one without a workspace.
 hipError_t launch_fmha_prefill(const void* q, const void* k_cache, const void* v_cache,
                                void* out, int seq_len, int pos0, int Hq, int Hkv,
-                               long head_stride, float qk_scale, hipStream_t stream);
+                               long head_stride, float qk_scale, hipStream_t stream,
+                               void* workspace = nullptr, size_t workspace_bytes = 0);
 
 // Model-step kernels (model_kernels.hip).  residual == nullptr selects plain
 // RMSNorm; otherwise out = norm(residual + x), residual_out = residual + x.

@@ -104,6 +104,15 @@ def fmha_prefill(q, k_cache, v_cache, position_start: int, out=None,
     out = torch.empty_like(q) if out is None else out
     _f16(out, "out", (S, Hq, D))
     qk_scale = 1.0 / math.sqrt(D) if qk_scale is None else qk_scale
+    # up to 24 kv tiles of 64 positions the kv range is never split
+    nbytes = 0 if position_start + S <= 1536 else int(
+        lib().grout_fmha_prefill_workspace_bytes(S, position_start, Hq, Hkv))
+    if nbytes:
+        ws = torch.empty(nbytes // 4, dtype=torch.float32, device=q.device)
+        call("grout_fmha_prefill_ws", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(ws),
+             nbytes, S, position_start, Hq, Hkv, D, k_cache.shape[1] * D, qk_scale,
+             _stream(q.device))
+        return out
     call("grout_fmha_prefill", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), S,
          position_start, Hq, Hkv, D, k_cache.shape[1] * D, qk_scale, _stream(q.device))
     return out

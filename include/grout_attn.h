@@ -110,6 +110,22 @@ int grout_fmha_prefill(const void* q, const void* k_cache, const void* v_cache, 
                        int seq_len, int pos0, int num_q_heads, int num_kv_heads, int head_dim,
                        long kv_head_stride, float qk_scale, void* stream);
 
+/* Bytes of fp32 scratch with which a chunk of seq_len rows at pos0 runs fastest
+ * (host only; 0 when it needs none, or for invalid arguments).  A short chunk
+ * on a long cache has too few q blocks to fill the GPU: grout_fmha_prefill_ws
+ * then splits the kv range as well and merges the partials. */
+size_t grout_fmha_prefill_workspace_bytes(int seq_len, int pos0, int num_q_heads,
+                                          int num_kv_heads);
+
+/* grout_fmha_prefill with scratch (16-byte aligned device memory, may be NULL):
+ * as many kv ranges as workspace_bytes holds, at most what
+ * grout_fmha_prefill_workspace_bytes asks for; more than one adds a merge
+ * launch.  Calls sharing one workspace must not overlap in time. */
+int grout_fmha_prefill_ws(const void* q, const void* k_cache, const void* v_cache, void* out,
+                          void* workspace, size_t workspace_bytes, int seq_len, int pos0,
+                          int num_q_heads, int num_kv_heads, int head_dim, long kv_head_stride,
+                          float qk_scale, void* stream);
+
 /* The work split grout_fmha_prefill launches for seq_len query rows (host
  * only, no GPU; the GROUT_FMHA_PREFILL_SHARED / _PAIRED / _WAVE_ROWS test
  * overrides apply): *form = 0 the shared K/V stream (256-row q blocks), 1 the

@@ -399,3 +399,17 @@ def test_low_bit_k_limit_covers_qwen3_without_gpu():
         for k in (17408, 25600, 32768):
             assert L.grout_qweight_bytes(fmt, 5120, k) > 0, (fmt, k)
         assert L.grout_qweight_bytes(fmt, 5120, 32768 + blk) == 0, fmt
+
+
+def test_prefill_workspace_rule():
+    """Only a chunk whose q blocks leave CUs idle on a long cache asks for
+    scratch; at most 16 ranges; none for invalid arguments."""
+    f = grout_amd.lib().grout_fmha_prefill_workspace_bytes
+    per = lambda S, Hq: S * Hq * 130 * 4
+    assert f(61, 8131, 32, 8) == 8 * per(61, 32)   # 32 workgroups x 8 fill the 256 CUs
+    assert f(1, 8000, 32, 8) == 16 * per(1, 32)
+    assert f(61, 0, 32, 8) == 0 and f(61, 1475, 32, 8) == 0 and f(61, 1476, 32, 8) > 0
+    assert f(500, 16000, 32, 8) == 0               # 256 workgroups already
+    assert f(2048, 8000, 32, 8) == 0
+    assert f(0, 100, 32, 8) == 0 and f(8, -1, 32, 8) == 0 and f(8, 4000, 33, 8) == 0
+    assert f(8, 1 << 22, 32, 8) == 0
