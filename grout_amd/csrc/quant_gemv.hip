@@ -16,13 +16,16 @@
 //   Q5_K: q and h as Q4_K, qh u8 [N][K/8] (each superblock's 32 qh bytes)
 //   Q6_K: ql u8 [N][K/2], qh u8 [N][K/4], sc int8 [N][K/16], d f16 [N][K/256]
 //
-// GEMV kernel: one 16-lane team per weight row, x and the rows' decoded
-// block scales staged in LDS (swizzled against bank conflicts), the weights
-// streamed with every load of a lane in flight before its first use.  A run
-// of 16 quantized values becomes exact f16 integers (v_perm inserts 0x64, the
-// exponent byte of 1024, above each byte; a packed subtract removes 1024 plus
-// the format's offset), its dot product with x uses v_dot2_f32_f16, and the
-// run's scale (and min) is applied once: scale * sum(q x) - min * sum(x).
+// GEMV kernel: one 16-lane team per weight row (or two), x and the rows'
+// decoded block scales staged in LDS (swizzled against bank conflicts), the
+// weights streamed with every load of a lane in flight before its first use.
+// A run of 16 quantized values becomes exact f16 denormals (v_perm puts a zero
+// byte above each byte: byte * 2^-24), its dot product with x uses
+// v_dot2_f32_f16, and the run's scale (and min) is applied once: scale *
+// sum(q x) - min * sum(x).  At the layer shapes the time is VALU work as much
+// as bytes: of ~1000 instructions a thread ran for Qwen3-4B's Q4_K gate_up with
+// its norm, 330 were the dot and 500 the staging of x and scales (10.2 us; 9.5
+// with 700).
 #include "common.hpp"
 #include "kernels.hpp"
 #include "quant_layout.hpp"
@@ -84,9 +87,8 @@ __global__ __launch_bounds__(256) void qrepack_kernel(int fmt, const uint8_t* __
 
 // ---------------------------------------------------------------- GEMV
 //
-// A row team of 16 lanes owns one weight row; lane m takes the row's pieces
-// p = m, m + 16, ... (a piece is 32 consecutive weights: Q8_0 one block;
-// Q4_K 16 qs bytes = 16 weights of sub-block 2g in the low nibbles and 16 of
+// A row team of 16 lanes owns one weight row (RPT = 2: two); lane m takes the
+// row's pieces p = m, m + 16, ... (a piece is 32 weights: Q8_0 one block; Q4_K 16 qs bytes = 16 weights of sub-block 2g in the low nibbles and 16 of
 // 2g+1 in the high; Q5_K the same and the 16 qh bytes holding their fifth
 // bits; Q6_K 16 ql bytes and the 16 qh bytes they pair with), so a
 // team reads 256 contiguous bytes per load and p % 8 == m % 8 fixes each
@@ -128,17 +130,24 @@ __host__ __device__ constexpr int xswz(int G) {
 __host__ __device__ constexpr int xsum_slot(int r) { return (r & ~3) | ((r & 1) << 1) | ((r >> 1) & 1); }
 __host__ __device__ constexpr int q6_slot(int r) { return (r & ~7) | ((r & 3) << 1) | ((r >> 2) & 1); }
 
-// Weight row of local row lr and the output it feeds.  SILU: in each wave the
-// teams are gate rows o, o+1 then the up rows o, o+1 (up row = N + o).
-template <bool SILU, int R>
+// Weight row of local row lr (of R RPT in the workgroup) and the output it
+// feeds.  SILU: with one row per team, each wave's teams are gate rows o, o+1
+// then the up rows o, o+1 (up row = N + o); with two, a team owns gate row o
+// and up row N + o.
+template <bool SILU, int R, int RPT>
 __device__ __forceinline__ int qrow(int lr, int N, int& out) {
-  if (SILU) {
+  if (SILU && RPT == 1) {
     const int t = lr & 3;
     out = (int)blockIdx.x * (R / 2) + 2 * (lr >> 2) + (t & 1);
     const int o = min(out, N - 1);
     return t < 2 ? o : N + o;
   }
-  out = (int)blockIdx.x * R + lr;
+  if (SILU) {
+    out = (int)blockIdx.x * R + (lr >> 1);
+    const int o = min(out, N - 1);
+    return (lr & 1) ? N + o : o;
+  }
+  out = (int)blockIdx.x * (R * RPT) + lr;
   return min(out, N - 1);
 }
 
@@ -238,7 +247,7 @@ __device__ __forceinline__ half8 xgran(const unsigned char* s_xb, int off) {
 }
 
 // Contribution of piece i of lane m (piece index p = m + 16 i) to the row's
-// dot product.  Staged scales carry the 2^24 of the denormal encoding.
+// dot product (Q4_K, Q5_K: times 2^-24, the denormal encoding).
 template <int FMT, int I>
 __device__ __forceinline__ float qpc_dot(const QPc& r, int m, const QLane& q,
                                          const unsigned char* s_xb, const float* s_xsum,
@@ -261,7 +270,7 @@ __device__ __forceinline__ float qpc_dot(const QPc& r, int m, const QLane& q,
     }
     const float dlo = ddot16(lo, xgran<I>(s_xb, q.xg[0]), xgran<I>(s_xb, q.xg[1]), 0.f);
     const float dhi = ddot16(hi, xgran<I>(s_xb, q.xg[2]), xgran<I>(s_xb, q.xg[3]), 0.f);
-    // {2^24 d sc_2g, dmin m_2g, 2^20 d sc_2g+1, dmin m_2g+1}
+    // {d sc_2g, dmin m_2g, 2^-4 d sc_2g+1, dmin m_2g+1}
     const floatx4 sc = *reinterpret_cast<const floatx4*>(s_row + q.so + 32 * I);
     const float2 xs = *reinterpret_cast<const float2*>(s_xsum + q.xo + 32 * I);
     return (sc[0] * dlo - sc[1] * xs.x) + (sc[2] * dhi - sc[3] * xs.y);
@@ -277,7 +286,7 @@ __device__ __forceinline__ float qpc_dot(const QPc& r, int m, const QLane& q,
     }
     const float dlo = ddot16(lo, xgran<I>(s_xb, q.xg[0]), xgran<I>(s_xb, q.xg[1]), 0.f);
     const float dhi = ddot16(hi, xgran<I>(s_xb, q.xg[2]), xgran<I>(s_xb, q.xg[3]), 0.f);
-    // {2^24 d sc_2g, dmin m_2g, 2^24 d sc_2g+1, dmin m_2g+1}
+    // {d sc_2g, dmin m_2g, d sc_2g+1, dmin m_2g+1}
     const floatx4 sc = *reinterpret_cast<const floatx4*>(s_row + q.so + 32 * I);
     const float2 xs = *reinterpret_cast<const float2*>(s_xsum + q.xo + 32 * I);
     return (sc[0] * dlo - sc[1] * xs.x) + (sc[2] * dhi - sc[3] * xs.y);
@@ -298,9 +307,9 @@ __device__ __forceinline__ float qpc_dot(const QPc& r, int m, const QLane& q,
   }
 }
 
-// Staging of x: granule c to its swizzled slot, and the x sum of each run
-// (Q8_0: 32-runs = granules c..c+3, scaled by 128 * 2^-24; Q4_K, Q5_K: 16-runs;
-// Q6_K: 16-runs scaled by 32 * 2^-24), the run's granules sitting in
+// Staging of x: granule c to its swizzled slot, and the x sum of each run, in
+// the denormal encoding's 2^-24 (Q8_0: 32-runs = granules c..c+3, times 128;
+// Q4_K, Q5_K: 16-runs; Q6_K: 16-runs times 32), the run's granules sitting in
 // adjacent lanes.  Every lane calls it.
 template <int FMT>
 __device__ __forceinline__ void stage_x(u32x4 v, int c, int NG, half_t* s_x, float* s_xsum) {
@@ -314,7 +323,7 @@ __device__ __forceinline__ void stage_x(u32x4 v, int c, int NG, half_t* s_x, flo
     s += xor_lane<2>(s);
     if (c < NG && (c & 3) == 0) s_xsum[c >> 2] = s * 0x1p-17f;
   } else if (FMT == 12 || FMT == 13) {
-    if (c < NG && (c & 1) == 0) s_xsum[xsum_slot(c >> 1)] = s;
+    if (c < NG && (c & 1) == 0) s_xsum[xsum_slot(c >> 1)] = s * 0x1p-24f;
   } else {
     if (c < NG && (c & 1) == 0) s_xsum[q6_slot(c >> 1)] = s * 0x1p-19f;
   }
@@ -336,12 +345,12 @@ __device__ __forceinline__ int unit_row(int u, float inv_upr) {
   return (int)(((float)u + 0.5f) * inv_upr);
 }
 
-template <int FMT, bool SILU, int R>
+template <int FMT, bool SILU, int R, int RPT>
 __device__ __forceinline__ SRaw stage_load(const uint8_t* __restrict__ W, const QLayout& L, int u,
                                            int UPR, float inv_upr, int N, int K) {
   const int lr = unit_row(u, inv_upr), k = u - lr * UPR;
   int o;
-  const int row = qrow<SILU, R>(lr, N, o);
+  const int row = qrow<SILU, R, RPT>(lr, N, o);
   SRaw s;
   s.v = u32x4{0u, 0u, 0u, 0u};
   s.d = 0;
@@ -358,48 +367,43 @@ __device__ __forceinline__ SRaw stage_load(const uint8_t* __restrict__ W, const 
 
 // Scales as the reference's decode layout holds them (Q8_0 d; Q6_K d * sc in
 // fp32; Q4_K the effective f16(d * sc) and f16(dmin * m); Q5_K, read in the
-// native layout, d * sc and dmin * m in fp32), times the power of two that
-// undoes the denormal encoding (exact).
+// native layout, d * sc and dmin * m in fp32).  The power of two that undoes
+// the denormal encoding is exact wherever it is applied: in the Q8_0 and Q6_K
+// scales, and for Q4_K and Q5_K, with two numbers per 32 weights, in the
+// finished sum.
 template <int FMT>
 __device__ __forceinline__ void stage_store(const SRaw& s, int u, int U, int UPR, float inv_upr,
                                             int SCW, float* s_sc) {
   if (u >= U) return;
   const int lr = unit_row(u, inv_upr), k = u - lr * UPR;
   float* dst = s_sc + lr * SCW;
+  auto byte = [](uint32_t w, int i) __attribute__((always_inline)) {
+    return (float)((w >> (8 * i)) & 0xffu);  // v_cvt_f32_ubyte
+  };
   if (FMT == 8) {
     dst[k] = h2f_bits((uint16_t)s.d) * 0x1p24f;
   } else if (FMT == 12 || FMT == 13) {
-    // d, dmin, then eight 6-bit (scale, min) pairs packed in 12 bytes
+    // d, dmin, then eight 6-bit (scale, min) pairs packed in 12 bytes: four at
+    // a time, sub-blocks 0-3 and 4-7
     const float d = h2f_bits((uint16_t)(s.v[0] & 0xFFFFu));
     const float dmin = h2f_bits((uint16_t)(s.v[0] >> 16));
-    int q[12];
+    const uint32_t sc[2] = {s.v[1] & 0x3f3f3f3fu,
+                            (s.v[3] & 0x0f0f0f0fu) | ((s.v[1] >> 2) & 0x30303030u)};
+    const uint32_t mn[2] = {s.v[2] & 0x3f3f3f3fu,
+                            ((s.v[3] >> 4) & 0x0f0f0f0fu) | ((s.v[2] >> 2) & 0x30303030u)};
 #pragma unroll
-    for (int j = 0; j < 12; ++j) q[j] = (s.v[1 + j / 4] >> (8 * (j % 4))) & 0xFF;
-    int sc[8], mn[8];
+    for (int g = 0; g < 4; ++g) {  // sub-blocks 2g, 2g + 1
+      const uint32_t ws = sc[g >> 1], wm = mn[g >> 1];
+      const int i = 2 * (g & 1);
+      // the products are exact in fp32 (11-bit d times a 6-bit integer)
+      floatx4 o = {d * byte(ws, i), dmin * byte(wm, i), d * byte(ws, i + 1),
+                   dmin * byte(wm, i + 1)};
+      if (FMT == 12) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j < 4) {
-        sc[j] = q[j] & 63;
-        mn[j] = q[j + 4] & 63;
-      } else {
-        sc[j] = (q[j + 4] & 0xF) | ((q[j - 4] >> 6) << 4);
-        mn[j] = (q[j + 4] >> 4) | ((q[j] >> 6) << 4);
+        for (int e = 0; e < 4; ++e) o[e] = (float)(half_t)o[e];
+        o[2] *= 0x1p-4f;  // the high nibbles are summed as 16 q
       }
-    }
-    if (FMT == 12) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<floatx4*>(dst + 16 * k + 4 * g) =
-            floatx4{(float)f2h_signed(d * (float)sc[2 * g]) * 0x1p24f,
-                    (float)f2h_signed(dmin * (float)mn[2 * g]),
-                    (float)f2h_signed(d * (float)sc[2 * g + 1]) * 0x1p20f,
-                    (float)f2h_signed(dmin * (float)mn[2 * g + 1])};
-    } else {  // the products are exact in fp32 (11-bit d times a 6-bit integer)
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<floatx4*>(dst + 16 * k + 4 * g) =
-            floatx4{(d * (float)sc[2 * g]) * 0x1p24f, dmin * (float)mn[2 * g],
-                    (d * (float)sc[2 * g + 1]) * 0x1p24f, dmin * (float)mn[2 * g + 1]};
+      *reinterpret_cast<floatx4*>(dst + 16 * k + 4 * g) = o;
     }
   } else {
     const float d = h2f_bits((uint16_t)s.d);
@@ -421,21 +425,29 @@ constexpr int qbatch() {
   return NPW > 0 && NPW < cap ? NPW : cap;
 }
 
-// Consumes pieces st + J.. of the lane's slice (counted from piece i0 on),
-// refilling each slot B pieces ahead.
-template <int FMT, int NPW, int B, int J>
-__device__ __forceinline__ void qconsume(QPc (&raw)[B], float& acc, int st, int i0, int m,
-                                         const QLane& q, const unsigned char* s_xb,
-                                         const float* s_xsum, const float* s_row,
-                                         const uint8_t* __restrict__ W, const QLayout& L, int row,
-                                         int K) {
+// Consumes pieces st + J.. of the lane's slice (counted from piece i0 on) of
+// its RPT rows, refilling each slot B pieces ahead.
+template <int FMT, int NPW, int B, int RPT, int J>
+__device__ __forceinline__ void qconsume(QPc (&raw)[B][RPT], float (&acc)[RPT], int st, int i0,
+                                         int m, const QLane& q, const unsigned char* s_xb,
+                                         const float* s_xsum, const float* s_row, int scw,
+                                         const uint8_t* __restrict__ W, const QLayout& L,
+                                         const int (&row)[RPT], int K) {
   if constexpr (J < NPW) {
     // the LDS offsets of piece st + J are compile-time steps from the base
     // pointers, which already point at piece st
-    const float v = qpc_dot<FMT, J>(raw[J % B], m, q, s_xb, s_xsum, s_row);
-    acc += st + J >= i0 ? v : 0.f;
-    if constexpr (J + B < NPW) raw[J % B] = qpc_load<FMT>(W, L, row, m + 16 * (st + J + B), K);
-    qconsume<FMT, NPW, B, J + 1>(raw, acc, st, i0, m, q, s_xb, s_xsum, s_row, W, L, row, K);
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) {
+      const float v = qpc_dot<FMT, J>(raw[J % B][r], m, q, s_xb, s_xsum, s_row + r * scw);
+      acc[r] += st + J >= i0 ? v : 0.f;
+    }
+    if constexpr (J + B < NPW) {
+#pragma unroll
+      for (int r = 0; r < RPT; ++r)
+        raw[J % B][r] = qpc_load<FMT>(W, L, row[r], m + 16 * (st + J + B), K);
+    }
+    qconsume<FMT, NPW, B, RPT, J + 1>(raw, acc, st, i0, m, q, s_xb, s_xsum, s_row, scw, W, L, row,
+                                      K);
   }
 }
 
@@ -457,14 +469,27 @@ __device__ half_t kQZero[kQMaxK];
 
 __device__ __forceinline__ float qwave_sum(float v) { return wave_xor_sum(v); }
 
-// c of chunk (8 values) and its contribution to sum(c^2).
+// a + b of two f16 halves in fp32 with one instruction (fma(a, 1, b), both
+// operands widened exactly): half HI of each word.
+template <bool HI>
+__device__ __forceinline__ float add_halves(uint32_t a, uint32_t b) {
+  float r;
+  if constexpr (HI)
+    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(r) : "v"(a), "v"(b));
+  else
+    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,1]" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// c of a chunk (8 values) and its contribution to sum(c^2).
 __device__ __forceinline__ float qnorm_c(u32x4 xv, u32x4 rv, float (&c)[8]) {
-  const half8 xh = as_half8(xv), rh = as_half8(rv);
   float part = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    c[e] = (float)rh[e] + (float)xh[e];
-    part += c[e] * c[e];
+  for (int e = 0; e < 4; ++e) {
+    c[2 * e] = add_halves<false>(xv[e], rv[e]);
+    c[2 * e + 1] = add_halves<true>(xv[e], rv[e]);
+    part += c[2 * e] * c[2 * e];
+    part += c[2 * e + 1] * c[2 * e + 1];
   }
   return part;
 }
@@ -482,36 +507,37 @@ __device__ __forceinline__ float qnorm_inv(float ss, int K, float eps, float* s_
   return 1.0f / sqrtf(ss / (float)K + eps);
 }
 
-// x' of one chunk; the first workgroup also writes f16(c) to residual_out.
-__device__ __forceinline__ u32x4 qnorm_apply(u32x4 xv, u32x4 rv, u32x4 gv, float inv, int c, int NG,
-                                             const QNorm& nz) {
-  float cv[8];
-  (void)qnorm_c(xv, rv, cv);
+// x' of one chunk from its c; the first workgroup also writes f16(c) to
+// residual_out.
+__device__ __forceinline__ u32x4 qnorm_apply(const float (&cv)[8], u32x4 gv, float inv, int c,
+                                             int NG, const QNorm& nz) {
   const half8 gh = as_half8(gv);
-  half8 o, co;
+  half8 o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    o[e] = (half_t)(cv[e] * inv * (float)gh[e]);
-    co[e] = (half_t)cv[e];
-  }
-  if (nz.res_out != nullptr && blockIdx.x == 0 && c < NG)
+  for (int e = 0; e < 8; ++e) o[e] = (half_t)(cv[e] * inv * (float)gh[e]);
+  if (nz.res_out != nullptr && blockIdx.x == 0 && c < NG) {
+    half8 co;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) co[e] = (half_t)cv[e];
     *reinterpret_cast<u32x4*>(nz.res_out + 8 * c) = as_u32x4(co);
+  }
   return as_u32x4(o);
 }
 
-// R weight rows per workgroup, each split into S slices of NPW pieces per
-// lane (one slice per group of R teams; K a multiple of 512 with
+// R teams of RPT weight rows per workgroup, each row split into S slices of NPW
+// pieces per lane (one slice per group of R teams; K a multiple of 512 with
 // NPW * S >= K / 512 >= NPW), or NPW = 0: any K, S = 1.  NORM: x is the
 // RMSNorm of residual + x (QNorm).
-template <int FMT, bool SILU, int R, int S, int NPW, bool NORM>
+template <int FMT, bool SILU, int R, int S, int NPW, bool NORM, int RPT>
 __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* __restrict__ W,
                                                                const half_t* __restrict__ x,
                                                                half_t* __restrict__ y, int N,
                                                                int K, QLayout L, QNorm nz) {
   constexpr int T = R * S * kQTeam;
   constexpr int B = qbatch<FMT, R, NPW>();
+  constexpr int RW = R * RPT;  // weight rows of the workgroup
   // LDS: x (K halves, padded to whole swizzle runs), x sums, each local row's
-  // scales (SCW floats), then S x R slice partials and one float per wave
+  // scales (SCW floats), then S x RW slice partials and one float per wave
   // for the norm.
   extern __shared__ __attribute__((aligned(16))) unsigned char s_dyn[];
   const int KX = (K + 127) & ~127;
@@ -521,19 +547,22 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
   const int SCW = FMT == 8 ? K / 32 : K / 16;
   const int UPR = FMT == 8 ? K / 32 : K / 256;  // staging units per row
   const float inv_upr = __builtin_amdgcn_rcpf((float)UPR);
-  const int U = R * UPR, NG = K / 8, P = K / 32;
+  const int U = RW * UPR, NG = K / 8, P = K / 32;
   const int tid = threadIdx.x, slice = tid / (R * kQTeam), team = (tid >> 4) % R, m = tid & 15;
-  int out;
-  const int row = qrow<SILU, R>(team, N, out);
-  const float* const s_row = s_sc + team * SCW;
+  int out[RPT], row[RPT];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) row[r] = qrow<SILU, R, RPT>(team * RPT + r, N, out[r]);
+  const float* const s_row = s_sc + team * RPT * SCW;
   const QLane q = qlane<FMT>(m);
-  float acc = 0.f;
+  float acc[RPT];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) acc[r] = 0.f;
 
   if constexpr (NPW > 0) {
     // x, scale and first weight loads all in flight before any is used (the
     // per-thread counts are bounds: NP <= NPW * S pieces per lane)
     constexpr int NXJ = (NPW * S * 64 + T - 1) / T;
-    constexpr int NUJ = ((FMT == 8 ? 16 : 2) * R * NPW * S + T - 1) / T;
+    constexpr int NUJ = ((FMT == 8 ? 16 : 2) * RW * NPW * S + T - 1) / T;
     const int NP = K / 512;
     // slice pieces i0 .. i0 + NPW - 1 clipped to NP: a slice that would run
     // past the end starts at NP - NPW and counts only pieces >= i0
@@ -551,32 +580,44 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
     SRaw ur[NUJ];
 #pragma unroll
     for (int j = 0; j < NUJ; ++j)
-      ur[j] = stage_load<FMT, SILU, R>(W, L, min(tid + T * j, U - 1), UPR, inv_upr, N, K);
-    QPc raw[B];
+      ur[j] = stage_load<FMT, SILU, R, RPT>(W, L, min(tid + T * j, U - 1), UPR, inv_upr, N, K);
+    QPc raw[B][RPT];
 #pragma unroll
-    for (int b = 0; b < B; ++b) raw[b] = qpc_load<FMT>(W, L, row, m + 16 * (st + b), K);
+    for (int b = 0; b < B; ++b)
+#pragma unroll
+      for (int r = 0; r < RPT; ++r)
+        raw[b][r] = qpc_load<FMT>(W, L, row[r], m + 16 * (st + b), K);
     __builtin_amdgcn_sched_barrier(0);
+    // chunks j of this wave past the end are skipped by the whole wave
+    const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63);
     if constexpr (NORM) {
-      float ss = 0.f;
+      float ss = 0.f, cv[8];
 #pragma unroll
       for (int j = 0; j < NXJ; ++j) {
-        float cv[8];
-        const float part = qnorm_c(xr[j], rr[j], cv);
-        ss += tid + T * j < NG ? part : 0.f;
+        if (wave0 + T * j < NG) {
+          const float part = qnorm_c(xr[j], rr[j], cv);
+          ss += tid + T * j < NG ? part : 0.f;
+        }
       }
-      const float inv = qnorm_inv<T>(ss, K, nz.eps, s_sc + R * SCW + S * R);
+      const float inv = qnorm_inv<T>(ss, K, nz.eps, s_sc + RW * SCW + S * RW);
 #pragma unroll
-      for (int j = 0; j < NXJ; ++j) xr[j] = qnorm_apply(xr[j], rr[j], gr[j], inv, tid + T * j, NG, nz);
+      for (int j = 0; j < NXJ; ++j) {
+        if (wave0 + T * j < NG) {  // c again: eight instructions, not eight live registers
+          (void)qnorm_c(xr[j], rr[j], cv);
+          xr[j] = qnorm_apply(cv, gr[j], inv, tid + T * j, NG, nz);
+        }
+      }
     }
 #pragma unroll
-    for (int j = 0; j < NXJ; ++j) stage_x<FMT>(xr[j], tid + T * j, NG, s_x, s_xsum);
+    for (int j = 0; j < NXJ; ++j)
+      if (!NORM || wave0 + T * j < NG) stage_x<FMT>(xr[j], tid + T * j, NG, s_x, s_xsum);
 #pragma unroll
     for (int j = 0; j < NUJ; ++j) stage_store<FMT>(ur[j], tid + T * j, U, UPR, inv_upr, SCW, s_sc);
     __syncthreads();
     const int fs = FMT == 8 ? 16 : 32;  // scale / x-sum floats per piece step
-    qconsume<FMT, NPW, B, 0>(raw, acc, st, i0, m, q,
-                             reinterpret_cast<const unsigned char*>(s_x) + 1024 * st,
-                             s_xsum + fs * st, s_row + fs * st, W, L, row, K);
+    qconsume<FMT, NPW, B, RPT, 0>(raw, acc, st, i0, m, q,
+                                  reinterpret_cast<const unsigned char*>(s_x) + 1024 * st,
+                                  s_xsum + fs * st, s_row + fs * st, SCW, W, L, row, K);
   } else {
     const int nxj = (NG + T - 1) / T;
     float inv = 0.f;
@@ -589,17 +630,20 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
         const float part = qnorm_c(load16(x + 8 * cc), load16(res + 8 * cc), cv);
         ss += c < NG ? part : 0.f;
       }
-      inv = qnorm_inv<T>(ss, K, nz.eps, s_sc + R * SCW + S * R);
+      inv = qnorm_inv<T>(ss, K, nz.eps, s_sc + RW * SCW + S * RW);
     }
     for (int j = 0; j < nxj; ++j) {
       const int c = tid + T * j, cc = min(c, NG - 1);
       u32x4 xv = load16(x + 8 * cc);
-      if constexpr (NORM)
-        xv = qnorm_apply(xv, load16(res + 8 * cc), load16(nz.gamma + 8 * cc), inv, c, NG, nz);
+      if constexpr (NORM) {
+        float cv[8];
+        (void)qnorm_c(xv, load16(res + 8 * cc), cv);
+        xv = qnorm_apply(cv, load16(nz.gamma + 8 * cc), inv, c, NG, nz);
+      }
       stage_x<FMT>(xv, c, NG, s_x, s_xsum);
     }
     for (int u = tid; u < U; u += T)
-      stage_store<FMT>(stage_load<FMT, SILU, R>(W, L, u, UPR, inv_upr, N, K), u, U, UPR, inv_upr,
+      stage_store<FMT>(stage_load<FMT, SILU, R, RPT>(W, L, u, UPR, inv_upr, N, K), u, U, UPR, inv_upr,
                        SCW, s_sc);
     __syncthreads();
     const int npl = (P + 15) / 16;
@@ -607,37 +651,57 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
     const unsigned char* s_xb = reinterpret_cast<const unsigned char*>(s_x);
     for (int i = 0; i < npl; ++i) {
       const int p = m + 16 * i;
-      const QPc r = qpc_load<FMT>(W, L, row, min(p, P - 1), K);
-      const float v = qpc_dot<FMT, 0>(r, m, q, s_xb + 1024 * i, s_xsum + fs * i, s_row + fs * i);
-      acc += p < P ? v : 0.f;
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) {
+        const QPc w = qpc_load<FMT>(W, L, row[r], min(p, P - 1), K);
+        const float v = qpc_dot<FMT, 0>(w, m, q, s_xb + 1024 * i, s_xsum + fs * i,
+                                        s_row + r * SCW + fs * i);
+        acc[r] += p < P ? v : 0.f;
+      }
     }
   }
 
   // the team's 16 lanes, butterfly order (lane ^ 8, 4, 2, 1), on the VALU
-  acc += xor_lane<8>(acc);
-  acc += xor_lane<4>(acc);
-  acc += xor_lane<2>(acc);
-  acc += xor_lane<1>(acc);
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    acc[r] += xor_lane<8>(acc[r]);
+    acc[r] += xor_lane<4>(acc[r]);
+    acc[r] += xor_lane<2>(acc[r]);
+    acc[r] += xor_lane<1>(acc[r]);
+  }
   if constexpr (S > 1) {
     // slice partials summed in slice order by slice 0
-    float* const s_red = s_sc + R * SCW;
-    if (m == 0) s_red[slice * R + team] = acc;
+    float* const s_red = s_sc + RW * SCW;
+    if (m == 0) {
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) s_red[slice * RW + team * RPT + r] = acc[r];
+    }
     __syncthreads();
     if (slice != 0) return;
-    acc = s_red[team];
 #pragma unroll
-    for (int w = 1; w < S; ++w) acc += s_red[w * R + team];
+    for (int r = 0; r < RPT; ++r) {
+      acc[r] = s_red[team * RPT + r];
+#pragma unroll
+      for (int w = 1; w < S; ++w) acc[r] += s_red[w * RW + team * RPT + r];
+    }
   }
-  if (SILU) {
-    const float up = xor_lane<32>(acc);  // gate teams 0, 1 <-> up teams 2, 3
-    if (m == 0 && (team & 3) < 2 && out < N) {
-      const half_t g = (half_t)acc, u = (half_t)up;
+  if constexpr (FMT == 12 || FMT == 13) {
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) acc[r] *= 0x1p24f;
+  }
+  if constexpr (SILU) {
+    // one row per team: gate teams 0, 1 <-> up teams 2, 3
+    const float up = RPT == 1 ? xor_lane<32>(acc[0]) : acc[RPT - 1];
+    if (m == 0 && (RPT == 2 || (team & 3) < 2) && out[0] < N) {
+      const half_t g = (half_t)acc[0], u = (half_t)up;
       const float gf = (float)g;
       const float sig = 1.0f / (1.0f + expf(-gf));
-      y[out] = (half_t)(sig * gf * (float)u);
+      y[out[0]] = (half_t)(sig * gf * (float)u);
     }
-  } else if (m == 0 && out < N) {
-    y[out] = (half_t)acc;
+  } else {
+#pragma unroll
+    for (int r = 0; r < RPT; ++r)
+      if (m == r && out[r] < N) y[out[r]] = (half_t)acc[r];
   }
 }
 
@@ -800,26 +864,28 @@ static bool npw_short(int v) {
   return v == 2 || v == 3 || v == 4 || v == 5 || v == 8 || v == 10 || v == 13;
 }
 
-template <int FMT, bool SILU, int R, int S, bool NORM>
+template <int FMT, bool SILU, int R, int S, bool NORM, int RPT>
 static void gemv_q_go(int npw, unsigned grid, size_t lds, const void* W, const void* x, void* y,
                       int N, int K, const QLayout& L, const QNorm& nz, hipStream_t stream) {
   const uint8_t* w = (const uint8_t*)W;
   const half_t* xi = (const half_t*)x;
   half_t* yo = (half_t*)y;
   constexpr int T = R * S * kQTeam;
-#define GROUT_QGO(V) \
+#define GROUT_QGO(V)                                                                          \
   case V:                                                                                     \
-    gemv_q_kernel<FMT, SILU, R, S, V, NORM><<<grid, T, lds, stream>>>(w, xi, yo, N, K, L, nz); \
+    gemv_q_kernel<FMT, SILU, R, S, V, NORM, RPT><<<grid, T, lds, stream>>>(w, xi, yo, N, K, L, \
+                                                                          nz);                \
     break;
   if constexpr (R == 16) {
     switch (npw) {
       GROUT_QGO(5) GROUT_QGO(8) GROUT_QGO(10) GROUT_QGO(16) GROUT_QGO(19)
       default:
-        gemv_q_kernel<FMT, SILU, R, 1, 0, NORM><<<grid, T, lds, stream>>>(w, xi, yo, N, K, L, nz);
+        gemv_q_kernel<FMT, SILU, R, 1, 0, NORM, RPT><<<grid, T, lds, stream>>>(w, xi, yo, N, K, L,
+                                                                              nz);
     }
   } else if constexpr (SILU || S == 0) {
-    gemv_q_kernel<FMT, SILU, R, 1, 0, NORM><<<grid, R * kQTeam, lds, stream>>>(w, xi, yo, N, K, L,
-                                                                             nz);
+    gemv_q_kernel<FMT, SILU, R, 1, 0, NORM, RPT><<<grid, R * kQTeam, lds, stream>>>(w, xi, yo, N,
+                                                                                   K, L, nz);
   } else {
     switch (npw) {
       GROUT_QGO(2) GROUT_QGO(3) GROUT_QGO(4) GROUT_QGO(5) GROUT_QGO(8) GROUT_QGO(10)
@@ -863,12 +929,27 @@ static hipError_t gemv_q_launch(const void* W, const void* x, void* y, int N, in
   const QLayout L = qlayout(FMT, (size_t)rows, (size_t)K);
   const int np = K % 512 == 0 ? K / 512 : 0;  // pieces per lane of a whole row
   if (rows >= 16 * 1024 && gemv_q_lds<FMT>(16, 1, K) <= 65536) {
-    // tall: 16 rows per workgroup (x staged once per 16 rows)
+    // tall: 16 teams per workgroup, x staged once for all their rows.  Two rows
+    // per team for Q4_K and Q5_K, whose time is VALU work (staging x and its
+    // norm, decoding scales): half the staging per row.  Same-box us, one row
+    // -> two: Q4_K lm_head 151936 x 2560 38.6 -> 37.0, 32B gate_up 30.4 -> 29.0;
+    // Q5_K lm_head 49.9 -> 46.4; Q8_0 is bound by its bytes and loses (gate_up
+    // 14.2 -> 14.9), Q6_K's lm_head too (49.8 -> 50.4 after its norm).
+    const int npw = npw_tall(np) ? np : 0;
+    if constexpr (FMT == 12 || FMT == 13) {
+      const size_t lds2 = gemv_q_lds<FMT>(32, 1, K);
+      if (lds2 <= 65536) {
+        const int per = silu ? 16 : 32;
+        const unsigned grid = (unsigned)((N + per - 1) / per);
+        if (silu) gemv_q_go<FMT, true, 16, 1, NORM, 2>(npw, grid, lds2, W, x, y, N, K, L, nz, stream);
+        else gemv_q_go<FMT, false, 16, 1, NORM, 2>(npw, grid, lds2, W, x, y, N, K, L, nz, stream);
+        return hipGetLastError();
+      }
+    }
     const int per = silu ? 8 : 16;
     const unsigned grid = (unsigned)((N + per - 1) / per);
-    const int npw = npw_tall(np) ? np : 0;
-    if (silu) gemv_q_go<FMT, true, 16, 1, NORM>(npw, grid, gemv_q_lds<FMT>(16, 1, K), W, x, y, N, K, L, nz, stream);
-    else gemv_q_go<FMT, false, 16, 1, NORM>(npw, grid, gemv_q_lds<FMT>(16, 1, K), W, x, y, N, K, L, nz, stream);
+    if (silu) gemv_q_go<FMT, true, 16, 1, NORM, 1>(npw, grid, gemv_q_lds<FMT>(16, 1, K), W, x, y, N, K, L, nz, stream);
+    else gemv_q_go<FMT, false, 16, 1, NORM, 1>(npw, grid, gemv_q_lds<FMT>(16, 1, K), W, x, y, N, K, L, nz, stream);
     return hipGetLastError();
   }
   // short: 4 rows per workgroup, each row split over S waves so that the grid
@@ -877,20 +958,38 @@ static hipError_t gemv_q_launch(const void* W, const void* x, void* y, int N, in
   if (gemv_q_lds<FMT>(4, 4, K) > qmax_lds()) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)((N + per - 1) / per);
   if (silu) {
-    gemv_q_go<FMT, true, 4, 0, NORM>(0, grid, gemv_q_lds<FMT>(4, 1, K), W, x, y, N, K, L, nz, stream);
+    gemv_q_go<FMT, true, 4, 0, NORM, 1>(0, grid, gemv_q_lds<FMT>(4, 1, K), W, x, y, N, K, L, nz, stream);
     return hipGetLastError();
   }
-  int S = 0, npw = 0;
-  if (np > 0) {
-    for (int s = grid >= 2048 ? 1 : grid >= 1024 ? 2 : 4; s <= 4 && S == 0; s *= 2) {
-      const int v = (np + s - 1) / s;
-      if (v <= np && npw_short(v)) S = s, npw = v;
+  // With a norm input, two rows per team and four slices from 4096 rows on
+  // (Q8_0: 8192): the norm is staged once per 8 rows by 256 threads (us: Q4_K 6144 x 2560 6.65 ->
+  // 5.83, 10240 x 5120 14.96 -> 10.78; Q6_K 7.54 -> 6.51, 21.5 -> 13.0; 1024 x
+  // 2560 3.2 -> 3.4).
+  if constexpr (NORM) {
+    const int v = (np + 3) / 4;
+    if (N >= (FMT == 8 ? 8192 : 4096) && np > 0 && npw_short(v) && gemv_q_lds<FMT>(8, 4, K) <= 65536) {
+      gemv_q_go<FMT, false, 4, 4, NORM, 2>(v, (unsigned)((N + 7) / 8), gemv_q_lds<FMT>(8, 4, K), W,
+                                          x, y, N, K, L, nz, stream);
+      return hipGetLastError();
     }
   }
-  if (S == 0) gemv_q_go<FMT, false, 4, 0, NORM>(0, grid, gemv_q_lds<FMT>(4, 1, K), W, x, y, N, K, L, nz, stream);
-  else if (S == 1) gemv_q_go<FMT, false, 4, 1, NORM>(npw, grid, gemv_q_lds<FMT>(4, 1, K), W, x, y, N, K, L, nz, stream);
-  else if (S == 2) gemv_q_go<FMT, false, 4, 2, NORM>(npw, grid, gemv_q_lds<FMT>(4, 2, K), W, x, y, N, K, L, nz, stream);
-  else gemv_q_go<FMT, false, 4, 4, NORM>(npw, grid, gemv_q_lds<FMT>(4, 4, K), W, x, y, N, K, L, nz, stream);
+  // Slices: enough of them for the waves, else (short K) as many as leave each
+  // lane two pieces or more; the looped kernel only when no count fits (0.6B
+  // QKV 4096 x 1024 4.8 -> 3.2 us, o_proj 1024 x 2048 5.0 -> 3.1).
+  int S = 0, npw = 0;
+  if (np > 0) {
+    const int want = grid >= 2048 ? 1 : grid >= 1024 ? 2 : 4;
+    auto fits = [&](int s) {
+      const int v = (np + s - 1) / s;
+      if (S == 0 && v <= np && npw_short(v)) S = s, npw = v;
+    };
+    for (int s = want; s <= 4; s *= 2) fits(s);
+    for (int s = want / 2; s >= 1; s /= 2) fits(s);
+  }
+  if (S == 0) gemv_q_go<FMT, false, 4, 0, NORM, 1>(0, grid, gemv_q_lds<FMT>(4, 1, K), W, x, y, N, K, L, nz, stream);
+  else if (S == 1) gemv_q_go<FMT, false, 4, 1, NORM, 1>(npw, grid, gemv_q_lds<FMT>(4, 1, K), W, x, y, N, K, L, nz, stream);
+  else if (S == 2) gemv_q_go<FMT, false, 4, 2, NORM, 1>(npw, grid, gemv_q_lds<FMT>(4, 2, K), W, x, y, N, K, L, nz, stream);
+  else gemv_q_go<FMT, false, 4, 4, NORM, 1>(npw, grid, gemv_q_lds<FMT>(4, 4, K), W, x, y, N, K, L, nz, stream);
   return hipGetLastError();
 }
 
