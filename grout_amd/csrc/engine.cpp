@@ -242,6 +242,11 @@ int project_rows(grout_engine* e, const Mat* m, int np, const void* x, uint16_t*
     out->splits = grout::tok_gemm_splits(rows, n, k);
     out->parts = parts;
   }
+  if (few && np == 2 && grout::tok_gemm_pair_ok(m[0].fmt, m[1].fmt))
+    return hip_status(
+        grout::launch_tok_gemm_pair(m[0].fmt, m[0].data, m[0].rows, m[1].fmt, m[1].data, m[1].rows,
+                                    x, y, parts, n, rows, k, out->splits, e->stream),
+        "tok_gemm_pair");
   int col = 0;
   for (int i = 0; i < np; ++i) {
     if (few) {

@@ -139,6 +139,12 @@ bool tok_gemm_ok(int fmt, int M, int N, int K);
 int tok_gemm_splits(int M, int N, int K);
 hipError_t launch_tok_gemm(int fmt, const void* W, const void* x, void* y, float* part, long ldy,
                            int M, int N, int K, int splits, hipStream_t stream);
+// Two matrices over the same x in one launch (a Q4_K or Q5_K one followed by
+// Q6_K rows): columns [0, Na) and [Na, Na + Nb) of y / part.
+bool tok_gemm_pair_ok(int fmt_a, int fmt_b);
+hipError_t launch_tok_gemm_pair(int fmt_a, const void* Wa, int Na, int fmt_b, const void* Wb,
+                                int Nb, const void* x, void* y, float* part, long ldy, int M,
+                                int K, int splits, hipStream_t stream);
 
 // Writes the 16x16 C fragment of A x B for A[i][k] = i*32+k (k < 32), B = I
 // padded, one float per (lane, element): used to confirm the MFMA lane layout.

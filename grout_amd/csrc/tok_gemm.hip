@@ -33,6 +33,8 @@
 #include "kernels.hpp"
 #include "quant_layout.hpp"
 
+#include <type_traits>
+
 namespace grout {
 
 namespace {
@@ -193,17 +195,21 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int FMT, int MT, int SUB>
-__global__ __launch_bounds__(kWaves * 64, 2) void tok_gemm_kernel(TokArgs A) {
 #ifdef __HIP_DEVICE_COMPILE__
+// LDS of a workgroup: two slots of x, and of f16 weights.
+constexpr int x_slot(int mt, int sub) { return sub * mt * 16 * kSubBytes; }
+constexpr int w_slot(int fmt, int sub) { return fmt == kF16 ? kWaves * sub * 4096 : 16; }
+
+template <int FMT, int MT, int SUB>
+__device__ __forceinline__ void tok_gemm_rows(const TokArgs& A, int row_group,
+                                              unsigned char (&s_x)[2][x_slot(MT, SUB)],
+                                              unsigned char (&s_w)[2][w_slot(FMT, SUB)]) {
   constexpr bool WL = FMT == kF16;  // weights through LDS
   constexpr int XI = SUB * MT;      // x staging: 1 KiB instructions per wave and step
-  __shared__ __attribute__((aligned(1024))) unsigned char s_x[2][SUB * MT * 16 * kSubBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char s_w[2][WL ? kWaves * SUB * 4096 : 16];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kb = lane >> 4;
-  const int row0 = ((int)blockIdx.x * kWaves + w) * 16;
+  const int row0 = (row_group * kWaves + w) * 16;
   const int t0 = (int)blockIdx.z * MT * 16;
   const int K = A.K, N = A.N;
   const int s0 = (int)blockIdx.y * A.subs, s1 = min(s0 + A.subs, K / kSub);
@@ -356,16 +362,43 @@ __global__ __launch_bounds__(kWaves * 64, 2) void tok_gemm_kernel(TokArgs A) {
       *reinterpret_cast<u32x2*>(A.y + (size_t)t * A.ldy + n) = __builtin_bit_cast(u32x2, o);
     }
   }
+}
+#endif
+
+template <int FMT, int MT, int SUB>
+__global__ __launch_bounds__(kWaves * 64, 2) void tok_gemm_kernel(TokArgs A) {
+#ifdef __HIP_DEVICE_COMPILE__
+  __shared__ __attribute__((aligned(1024))) unsigned char s_x[2][x_slot(MT, SUB)];
+  __shared__ __attribute__((aligned(1024))) unsigned char s_w[2][w_slot(FMT, SUB)];
+  tok_gemm_rows<FMT, MT, SUB>(A, (int)blockIdx.x, s_x, s_w);
 #endif
 }
 
-// Token tiles of 16 per workgroup: the fewest instantiated tiles that cover M
-// in blocks of at most kMaxTiles.
+// Two matrices over the same x in one grid, low-bit formats: row groups
+// [0, groups_a) of the first, the rest of the second.  The Q6_K V rows of a
+// Q4_K_M layer are 16 row groups: a launch of their own left most CUs idle
+// (Qwen3-4B, 131 tokens 9.2 us after the 16.3 us of Q and K).
+template <int FA, int FB, int MT, int SUB>
+__global__ __launch_bounds__(kWaves * 64, 2) void tok_gemm_pair_kernel(TokArgs A, TokArgs B,
+                                                                      int groups_a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  __shared__ __attribute__((aligned(1024))) unsigned char s_x[2][x_slot(MT, SUB)];
+  __shared__ __attribute__((aligned(1024))) unsigned char s_w[2][w_slot(FA, SUB)];
+  const int g = (int)blockIdx.x;
+  if (g < groups_a)
+    tok_gemm_rows<FA, MT, SUB>(A, g, s_x, s_w);
+  else
+    tok_gemm_rows<FB, MT, SUB>(B, g - groups_a, s_x, s_w);
+#endif
+}
+
+// Token tiles of 16 per workgroup: the fewest that cover M in blocks of at
+// most kMaxTiles.
 constexpr int kMaxTiles = 10;
 int tiles_for(int M) {
   const int all = (M + 15) / 16, blocks = (all + kMaxTiles - 1) / kMaxTiles;
   const int mt = (all + blocks - 1) / blocks;
-  return mt <= 4 ? mt : mt <= 6 ? 6 : mt <= 8 ? 8 : 10;
+  return mt;
 }
 
 }  // namespace
@@ -394,40 +427,56 @@ int tok_gemm_splits(int M, int N, int K) {
   return (units + per - 1) / per;
 }
 
-template <int FMT, int MT, int SUB>
-static void tok_launch(const TokArgs& a, int splits, hipStream_t stream) {
-  const dim3 grid((unsigned)((a.N + kRowsPerWg - 1) / kRowsPerWg), (unsigned)splits,
-                  (unsigned)((a.M + 16 * MT - 1) / (16 * MT)));
-  tok_gemm_kernel<FMT, MT, SUB><<<grid, kWaves * 64, 0, stream>>>(a);
-}
+static unsigned row_groups(int N) { return (unsigned)((N + kRowsPerWg - 1) / kRowsPerWg); }
 
-template <int FMT>
-static hipError_t tok_launch_fmt(const TokArgs& a, int splits, hipStream_t stream) {
-  // SUB: two sub-steps per barrier while x stays small (low-bit only: with f16
-  // weights in LDS as well, one workgroup per CU would be left)
-  switch (tiles_for(a.M)) {
-    case 1: tok_launch<FMT, 1, FMT == kF16 ? 1 : 2>(a, splits, stream); break;
-    case 2: tok_launch<FMT, 2, FMT == kF16 ? 1 : 2>(a, splits, stream); break;
-    case 3: tok_launch<FMT, 3, 1>(a, splits, stream); break;
-    case 4: tok_launch<FMT, 4, 1>(a, splits, stream); break;
-    case 6: tok_launch<FMT, 6, 1>(a, splits, stream); break;
-    case 8:
-      if constexpr (FMT != kF16) { tok_launch<FMT, 8, 1>(a, splits, stream); break; }
-      return hipErrorInvalidValue;
-    case 10:
-      if constexpr (FMT != kF16) { tok_launch<FMT, 10, 1>(a, splits, stream); break; }
-      return hipErrorInvalidValue;
-    default:
-      return hipErrorInvalidValue;
+// SUB for MT token tiles: two sub-steps per barrier while x stays small
+// (low-bit only: with f16 weights in LDS as well, one workgroup per CU would
+// be left).
+template <int FMT, int MT>
+constexpr int sub_steps() { return FMT != kF16 && MT <= 2 ? 2 : 1; }
+
+// Calls f(integral_constant<MT>) for the tile count of M tokens.
+template <class F>
+static hipError_t for_tiles(int M, F f) {
+  switch (tiles_for(M)) {
+#define GROUT_TILES(mt) case mt: f(std::integral_constant<int, mt>{}); break;
+    GROUT_TILES(1) GROUT_TILES(2) GROUT_TILES(3) GROUT_TILES(4) GROUT_TILES(5)
+    GROUT_TILES(6) GROUT_TILES(7) GROUT_TILES(8) GROUT_TILES(9) GROUT_TILES(10)
+#undef GROUT_TILES
+    default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-hipError_t launch_tok_gemm(int fmt, const void* W, const void* x, void* y, float* part, long ldy,
-                           int M, int N, int K, int splits, hipStream_t stream) {
+template <int FMT>
+static hipError_t tok_launch(const TokArgs& a, int splits, hipStream_t stream) {
+  return for_tiles(a.M, [&](auto t) {
+    constexpr int MT = decltype(t)::value;
+    if constexpr (FMT != kF16 || MT <= 6) {  // f16: at most 96 tokens
+      const dim3 grid(row_groups(a.N), (unsigned)splits, (unsigned)((a.M + 16 * MT - 1) / (16 * MT)));
+      tok_gemm_kernel<FMT, MT, sub_steps<FMT, MT>()><<<grid, kWaves * 64, 0, stream>>>(a);
+    }
+  });
+}
+
+template <int FA, int FB>
+static hipError_t tok_launch_pair(const TokArgs& a, const TokArgs& b, int splits,
+                                  hipStream_t stream) {
+  return for_tiles(a.M, [&](auto t) {
+    constexpr int MT = decltype(t)::value;
+    const unsigned ga = row_groups(a.N);
+    const dim3 grid(ga + row_groups(b.N), (unsigned)splits,
+                    (unsigned)((a.M + 16 * MT - 1) / (16 * MT)));
+    tok_gemm_pair_kernel<FA, FB, MT, sub_steps<FA, MT>()>
+        <<<grid, kWaves * 64, 0, stream>>>(a, b, (int)ga);
+  });
+}
+
+static bool tok_args(TokArgs& a, int fmt, const void* W, const void* x, void* y, float* part,
+                     long ldy, int M, int N, int K, int splits) {
   if (!tok_gemm_ok(fmt, M, N, K) || splits < 1 || (splits > 1 && part == nullptr) || ldy % 4)
-    return hipErrorInvalidValue;
-  TokArgs a{};
+    return false;
+  a = TokArgs{};
   a.W = (const uint8_t*)W;
   a.x = (const half_t*)x;
   a.y = (half_t*)y;
@@ -438,15 +487,36 @@ hipError_t launch_tok_gemm(int fmt, const void* W, const void* x, void* y, float
   a.ldy = ldy;
   const int units = (K / kSub + 1) / 2;
   a.subs = 2 * ((units + splits - 1) / splits);
-  if ((long)a.subs * (splits - 1) >= K / kSub) return hipErrorInvalidValue;  // an empty range
   if (fmt != 0) a.L = qlayout(fmt, (size_t)N, (size_t)K);
+  return (long)a.subs * (splits - 1) < K / kSub;  // no empty range
+}
+
+hipError_t launch_tok_gemm(int fmt, const void* W, const void* x, void* y, float* part, long ldy,
+                           int M, int N, int K, int splits, hipStream_t stream) {
+  TokArgs a;
+  if (!tok_args(a, fmt, W, x, y, part, ldy, M, N, K, splits)) return hipErrorInvalidValue;
   switch (fmt) {
-    case 0: return tok_launch_fmt<0>(a, splits, stream);
-    case 8: return tok_launch_fmt<8>(a, splits, stream);
-    case 12: return tok_launch_fmt<12>(a, splits, stream);
-    case 13: return tok_launch_fmt<13>(a, splits, stream);
-    default: return tok_launch_fmt<14>(a, splits, stream);
+    case 0: return tok_launch<0>(a, splits, stream);
+    case 8: return tok_launch<8>(a, splits, stream);
+    case 12: return tok_launch<12>(a, splits, stream);
+    case 13: return tok_launch<13>(a, splits, stream);
+    default: return tok_launch<14>(a, splits, stream);
   }
+}
+
+bool tok_gemm_pair_ok(int fmt_a, int fmt_b) { return (fmt_a == 12 || fmt_a == 13) && fmt_b == 14; }
+
+hipError_t launch_tok_gemm_pair(int fmt_a, const void* Wa, int Na, int fmt_b, const void* Wb,
+                                int Nb, const void* x, void* y, float* part, long ldy, int M,
+                                int K, int splits, hipStream_t stream) {
+  TokArgs a, b;
+  if (!tok_gemm_pair_ok(fmt_a, fmt_b) || Na % 4 ||
+      !tok_args(a, fmt_a, Wa, x, y, part, ldy, M, Na, K, splits) ||
+      !tok_args(b, fmt_b, Wb, x, y ? (half_t*)y + Na : nullptr, part ? part + Na : nullptr, ldy, M,
+                Nb, K, splits))
+    return hipErrorInvalidValue;
+  return fmt_a == 12 ? tok_launch_pair<12, 14>(a, b, splits, stream)
+                     : tok_launch_pair<13, 14>(a, b, splits, stream);
 }
 
 }  // namespace grout

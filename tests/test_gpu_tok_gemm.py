@@ -41,7 +41,7 @@ def matrix(fmt, n, k, seed, L):
 
 
 # one token tile and its edges, every instantiated tile count, two token blocks
-TOKENS = [2, 15, 16, 17, 33, 49, 64, 65, 97, 128, 129, 160, 161, 320, 321, 480]
+TOKENS = [2, 15, 16, 17, 33, 49, 64, 65, 96, 97, 113, 128, 129, 160, 161, 320, 321, 480]
 # rows: fewer than a workgroup's 64, a ragged last workgroup, whole ones;
 # K: one sub-step (Q8_0, f16), an odd number of them, one superblock, the
 # ranges' ragged end
@@ -93,6 +93,37 @@ def test_tok_gemm_rows_and_partial_sums(gpu, fmt, m):
             got = part[:, :, 8:8 + n].double().sum(0)
             assert ((got - ref).abs() <= bound).all()
             assert (part[:, :, :8] == 5).all() and (part[:, :, 8 + n:] == 5).all()
+
+
+PAIR = "_ZN5grout20launch_tok_gemm_pairEiPKviiS1_iS1_PvPfliiiP12ihipStream_t"
+
+
+@pytest.mark.parametrize("fmt", [O.Q4_K, O.Q5_K])
+@pytest.mark.parametrize("m", [2, 17, 33, 131, 161])
+@pytest.mark.parametrize("na,nb", [(192, 64), (100, 20), (4, 128)])
+def test_tok_gemm_pair_equals_two_launches(gpu, fmt, m, na, nb):
+    """A pair launch writes the same bits as one launch per matrix."""
+    from grout_amd import lib
+
+    L, k = lib(), 768
+    f, g = tok_gemm(L), getattr(L, PAIR)
+    g.restype = C.c_int
+    g.argtypes = [C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_int] + [C.c_void_p] * 3 \
+        + [C.c_long] + [C.c_int] * 3 + [C.c_void_p]
+    (wa, _), (wb, _) = matrix(fmt, na, k, 1, L), matrix(O.Q6_K, nb, k, 2, L)
+    x = torch.randn((m, k), dtype=torch.float16, device="cuda")
+    ld = na + nb
+    off = lambda t, n: C.c_void_p(t.data_ptr() + n * t.element_size())
+    for splits in (1, 3):
+        y, z = (torch.full((m, ld), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
+        p, q = (torch.full((splits, m, ld), 5.0, device="cuda") for _ in range(2))
+        assert f(fmt, ptr(wa), ptr(x), ptr(y), ptr(p), ld, m, na, k, splits, None) == 0
+        assert f(O.Q6_K, ptr(wb), ptr(x), off(y, na), off(p, na), ld, m, nb, k, splits, None) == 0
+        assert g(fmt, ptr(wa), na, O.Q6_K, ptr(wb), nb, ptr(x), ptr(z), ptr(q), ld, m, k, splits,
+                 None) == 0
+        assert torch.equal(y, z) and torch.equal(p, q)
+    assert g(O.Q6_K, ptr(wb), nb, O.Q6_K, ptr(wb), nb, ptr(x), ptr(z), ptr(q), ld, m, k, 1,
+             None) != 0
 
 
 def test_tok_gemm_refuses_what_it_does_not_cover(gpu):
