@@ -365,7 +365,15 @@ int record_decode_step(grout_engine* e) {
     const void* xin = l == 0 ? e->d(b.hidden) : e->d(b.ff_down);
     void* res_out = l == 0 ? nullptr : e->d(b.hidden);
     size_t row = 0;
-    for (int i = 0; i < w.nqkv; ++i) {
+    const bool pair = w.nqkv == 2 && grout::gemv_q_norm_pair_ok(w.qkv[0].fmt, w.qkv[1].fmt,
+                                                                w.qkv[0].rows, H);
+    if (pair)
+      GROUT_CHECK(hip_status(
+          grout::launch_gemv_q_norm_pair(w.qkv[0].fmt, w.qkv[0].data, w.qkv[0].rows,
+                                         w.qkv[1].fmt, w.qkv[1].data, w.qkv[1].rows, res, xin,
+                                         w.input_norm, res_out, c.rms_norm_eps, e->d(b.qkv), H, s),
+          "gemv_q_norm_pair"));
+    for (int i = 0; i < (pair ? 0 : w.nqkv); ++i) {
       GROUT_CHECK(mat_gemv_norm(e, w.qkv[i], res, xin, w.input_norm, res_out,
                                 e->d<uint16_t>(b.qkv) + row, H, false));
       row += (size_t)w.qkv[i].rows;

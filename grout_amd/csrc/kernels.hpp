@@ -123,6 +123,14 @@ hipError_t launch_gemv_q(int fmt, const void* W, const void* x, void* y, int N, 
 hipError_t launch_gemv_q_norm(int fmt, const void* W, const void* residual, const void* x,
                               const void* gamma, void* residual_out, float eps, void* y, int N,
                               int K, bool silu, hipStream_t stream);
+// launch_gemv_q_norm of two matrices over the same input in one launch (y of Na
+// then Nb rows): a Q4_K or Q5_K one of 4096 rows or more, then Q6_K rows, at
+// K = 2560 .. 6144.
+bool gemv_q_norm_pair_ok(int fmt_a, int fmt_b, int Na, int K);
+hipError_t launch_gemv_q_norm_pair(int fmt_a, const void* Wa, int Na, int fmt_b, const void* Wb,
+                                   int Nb, const void* residual, const void* x, const void* gamma,
+                                   void* residual_out, float eps, void* y, int K,
+                                   hipStream_t stream);
 // out[t] = row ids[t] of the N x K matrix as f16 (CPU dequantization rule).
 hipError_t launch_qgather(int fmt, const void* W, int N, int K, const uint32_t* ids, int rows,
                           void* out, hipStream_t stream);

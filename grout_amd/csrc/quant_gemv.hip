@@ -135,19 +135,19 @@ __host__ __device__ constexpr int q6_slot(int r) { return (r & ~7) | ((r & 3) <<
 // then the up rows o, o+1 (up row = N + o); with two, a team owns gate row o
 // and up row N + o.
 template <bool SILU, int R, int RPT>
-__device__ __forceinline__ int qrow(int lr, int N, int& out) {
+__device__ __forceinline__ int qrow(int bid, int lr, int N, int& out) {
   if (SILU && RPT == 1) {
     const int t = lr & 3;
-    out = (int)blockIdx.x * (R / 2) + 2 * (lr >> 2) + (t & 1);
+    out = bid * (R / 2) + 2 * (lr >> 2) + (t & 1);
     const int o = min(out, N - 1);
     return t < 2 ? o : N + o;
   }
   if (SILU) {
-    out = (int)blockIdx.x * R + (lr >> 1);
+    out = bid * R + (lr >> 1);
     const int o = min(out, N - 1);
     return (lr & 1) ? N + o : o;
   }
-  out = (int)blockIdx.x * (R * RPT) + lr;
+  out = bid * (R * RPT) + lr;
   return min(out, N - 1);
 }
 
@@ -346,11 +346,11 @@ __device__ __forceinline__ int unit_row(int u, float inv_upr) {
 }
 
 template <int FMT, bool SILU, int R, int RPT>
-__device__ __forceinline__ SRaw stage_load(const uint8_t* __restrict__ W, const QLayout& L, int u,
-                                           int UPR, float inv_upr, int N, int K) {
+__device__ __forceinline__ SRaw stage_load(const uint8_t* __restrict__ W, const QLayout& L, int bid,
+                                           int u, int UPR, float inv_upr, int N, int K) {
   const int lr = unit_row(u, inv_upr), k = u - lr * UPR;
   int o;
-  const int row = qrow<SILU, R, RPT>(lr, N, o);
+  const int row = qrow<SILU, R, RPT>(bid, lr, N, o);
   SRaw s;
   s.v = u32x4{0u, 0u, 0u, 0u};
   s.d = 0;
@@ -510,12 +510,12 @@ __device__ __forceinline__ float qnorm_inv(float ss, int K, float eps, float* s_
 // x' of one chunk from its c; the first workgroup also writes f16(c) to
 // residual_out.
 __device__ __forceinline__ u32x4 qnorm_apply(const float (&cv)[8], u32x4 gv, float inv, int c,
-                                             int NG, const QNorm& nz) {
+                                             int NG, const QNorm& nz, int bid) {
   const half8 gh = as_half8(gv);
   half8 o;
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = (half_t)(cv[e] * inv * (float)gh[e]);
-  if (nz.res_out != nullptr && blockIdx.x == 0 && c < NG) {
+  if (nz.res_out != nullptr && bid == 0 && c < NG) {
     half8 co;
 #pragma unroll
     for (int e = 0; e < 8; ++e) co[e] = (half_t)cv[e];
@@ -529,10 +529,9 @@ __device__ __forceinline__ u32x4 qnorm_apply(const float (&cv)[8], u32x4 gv, flo
 // NPW * S >= K / 512 >= NPW), or NPW = 0: any K, S = 1.  NORM: x is the
 // RMSNorm of residual + x (QNorm).
 template <int FMT, bool SILU, int R, int S, int NPW, bool NORM, int RPT>
-__global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* __restrict__ W,
-                                                               const half_t* __restrict__ x,
-                                                               half_t* __restrict__ y, int N,
-                                                               int K, QLayout L, QNorm nz) {
+__device__ __forceinline__ void gemv_q_rows(int bid, const uint8_t* __restrict__ W,
+                                            const half_t* __restrict__ x, half_t* __restrict__ y,
+                                            int N, int K, const QLayout& L, const QNorm& nz) {
   constexpr int T = R * S * kQTeam;
   constexpr int B = qbatch<FMT, R, NPW>();
   constexpr int RW = R * RPT;  // weight rows of the workgroup
@@ -551,7 +550,7 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
   const int tid = threadIdx.x, slice = tid / (R * kQTeam), team = (tid >> 4) % R, m = tid & 15;
   int out[RPT], row[RPT];
 #pragma unroll
-  for (int r = 0; r < RPT; ++r) row[r] = qrow<SILU, R, RPT>(team * RPT + r, N, out[r]);
+  for (int r = 0; r < RPT; ++r) row[r] = qrow<SILU, R, RPT>(bid, team * RPT + r, N, out[r]);
   const float* const s_row = s_sc + team * RPT * SCW;
   const QLane q = qlane<FMT>(m);
   float acc[RPT];
@@ -580,7 +579,7 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
     SRaw ur[NUJ];
 #pragma unroll
     for (int j = 0; j < NUJ; ++j)
-      ur[j] = stage_load<FMT, SILU, R, RPT>(W, L, min(tid + T * j, U - 1), UPR, inv_upr, N, K);
+      ur[j] = stage_load<FMT, SILU, R, RPT>(W, L, bid, min(tid + T * j, U - 1), UPR, inv_upr, N, K);
     QPc raw[B][RPT];
 #pragma unroll
     for (int b = 0; b < B; ++b)
@@ -604,7 +603,7 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
       for (int j = 0; j < NXJ; ++j) {
         if (wave0 + T * j < NG) {  // c again: eight instructions, not eight live registers
           (void)qnorm_c(xr[j], rr[j], cv);
-          xr[j] = qnorm_apply(cv, gr[j], inv, tid + T * j, NG, nz);
+          xr[j] = qnorm_apply(cv, gr[j], inv, tid + T * j, NG, nz, bid);
         }
       }
     }
@@ -638,12 +637,12 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
       if constexpr (NORM) {
         float cv[8];
         (void)qnorm_c(xv, load16(res + 8 * cc), cv);
-        xv = qnorm_apply(cv, load16(nz.gamma + 8 * cc), inv, c, NG, nz);
+        xv = qnorm_apply(cv, load16(nz.gamma + 8 * cc), inv, c, NG, nz, bid);
       }
       stage_x<FMT>(xv, c, NG, s_x, s_xsum);
     }
     for (int u = tid; u < U; u += T)
-      stage_store<FMT>(stage_load<FMT, SILU, R, RPT>(W, L, u, UPR, inv_upr, N, K), u, U, UPR, inv_upr,
+      stage_store<FMT>(stage_load<FMT, SILU, R, RPT>(W, L, bid, u, UPR, inv_upr, N, K), u, U, UPR, inv_upr,
                        SCW, s_sc);
     __syncthreads();
     const int npl = (P + 15) / 16;
@@ -702,6 +701,34 @@ __global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* _
 #pragma unroll
     for (int r = 0; r < RPT; ++r)
       if (m == r && out[r] < N) y[out[r]] = (half_t)acc[r];
+  }
+}
+
+template <int FMT, bool SILU, int R, int S, int NPW, bool NORM, int RPT>
+__global__ __launch_bounds__(R * S * kQTeam) void gemv_q_kernel(const uint8_t* __restrict__ W,
+                                                               const half_t* __restrict__ x,
+                                                               half_t* __restrict__ y, int N,
+                                                               int K, QLayout L, QNorm nz) {
+  gemv_q_rows<FMT, SILU, R, S, NPW, NORM, RPT>((int)blockIdx.x, W, x, y, N, K, L, nz);
+}
+
+// Two matrices over the same normed input in one grid (the Q and K rows of a
+// Q4_K_M layer, then its Q6_K V rows): workgroups [0, groups_a) take the
+// first.  A V launch of its own cost 3.3 us, most of it launch and staging of
+// the input norm: Qwen3-4B decode (36 layers) Q4_K_M 1263 -> 1203 us, Q5_K_M
+// 1372 -> 1310; 8 layers of Qwen3-32B Q4_K_M 734 -> 724.
+constexpr int kPairRows = 8;  // 4 teams of two rows, in four slices
+template <int FA, int FB, int NPW>
+__global__ __launch_bounds__(256) void gemv_q_norm_pair_kernel(
+    const uint8_t* __restrict__ Wa, const uint8_t* __restrict__ Wb, const half_t* __restrict__ x,
+    half_t* __restrict__ y, int Na, int Nb, int K, QLayout La, QLayout Lb, QNorm nz,
+    int groups_a) {
+  const int g = (int)blockIdx.x;
+  if (g < groups_a) {
+    gemv_q_rows<FA, false, 4, 4, NPW, true, 2>(g, Wa, x, y, Na, K, La, nz);
+  } else {
+    nz.res_out = nullptr;  // the first matrix's workgroup 0 writes it
+    gemv_q_rows<FB, false, 4, 4, NPW, true, 2>(g - groups_a, Wb, x, y + Na, Nb, K, Lb, nz);
   }
 }
 
@@ -1018,6 +1045,44 @@ hipError_t launch_gemv_q_norm(int fmt, const void* W, const void* residual, cons
       return norm ? gemv_q_launch<14, true>(W, x, y, N, K, silu, nz, stream)
                   : gemv_q_launch<14, false>(W, x, y, N, K, silu, nz, stream);
   }
+}
+
+// The forms in which the first matrix alone already runs as 4 teams of two rows
+// in 4 slices with its staging loads ahead in registers (gemv_q_launch's rule
+// for norm-folded rows), so its results stay bit for bit.
+bool gemv_q_norm_pair_ok(int fmt_a, int fmt_b, int Na, int K) {
+  const int v = (K / 512 + 3) / 4;
+  return (fmt_a == 12 || fmt_a == 13) && fmt_b == 14 && Na >= 4096 && K % 512 == 0 &&
+         (v == 2 || v == 3);
+}
+
+hipError_t launch_gemv_q_norm_pair(int fmt_a, const void* Wa, int Na, int fmt_b, const void* Wb,
+                                   int Nb, const void* residual, const void* x, const void* gamma,
+                                   void* residual_out, float eps, void* y, int K,
+                                   hipStream_t stream) {
+  if (!gemv_q_norm_pair_ok(fmt_a, fmt_b, Na, K) || Nb < 1 || gamma == nullptr)
+    return hipErrorInvalidValue;
+  const QNorm nz{(const half_t*)residual, (const half_t*)gamma, (half_t*)residual_out, eps};
+  const QLayout La = qlayout(fmt_a, (size_t)Na, (size_t)K), Lb = qlayout(fmt_b, (size_t)Nb, (size_t)K);
+  const unsigned ga = (unsigned)((Na + kPairRows - 1) / kPairRows);
+  const unsigned grid = ga + (unsigned)((Nb + kPairRows - 1) / kPairRows);
+  const size_t lds = gemv_q_lds<14>(kPairRows, 4, K);  // the K-quants stage alike
+  const uint8_t *wa = (const uint8_t*)Wa, *wb = (const uint8_t*)Wb;
+  const half_t* xi = (const half_t*)x;
+  half_t* yo = (half_t*)y;
+  const bool two = (K / 512 + 3) / 4 == 2;
+#define GROUT_PAIR(FA, NPW)                                                               \
+  gemv_q_norm_pair_kernel<FA, 14, NPW><<<grid, 256, lds, stream>>>(wa, wb, xi, yo, Na, Nb, \
+                                                                   K, La, Lb, nz, (int)ga)
+  if (fmt_a == 12) {
+    if (two) GROUT_PAIR(12, 2);
+    else GROUT_PAIR(12, 3);
+  } else {
+    if (two) GROUT_PAIR(13, 2);
+    else GROUT_PAIR(13, 3);
+  }
+#undef GROUT_PAIR
+  return hipGetLastError();
 }
 
 hipError_t launch_qgather(int fmt, const void* W, int N, int K, const uint32_t* ids, int rows,
