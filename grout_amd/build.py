@@ -32,12 +32,13 @@ SOURCES = [
     ("model_kernels.hip", []),
     ("quant_gemv.hip", []),
     ("tok_gemm.hip", []),
+    ("tile_gemm.hip", []),
     ("api.cpp", ["-x", "hip"]),
     ("engine.cpp", ["-x", "hip"]),
     ("loader.cpp", ["-x", "hip"]),
     ("gguf.cpp", ["-x", "hip"]),
 ]
-# Prefill projections are plain GEMMs: rocBLAS.
+# Projections of long prompts are plain GEMMs: rocBLAS.
 LIBS = ["-L/opt/rocm/lib", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"]
 
 

@@ -227,19 +227,22 @@ int mat_f16(grout_engine* e, const Mat& m, int k, const void** w) {
 // Projection of `rows` tokens by `np` parts (their rows follow each other)
 // into [rows][n] rows y, n the parts' rows in all.  A few tokens go through
 // the token GEMM, which may leave fp32 partial sums in `parts` instead of f16
-// rows (out says which); one token through the decode GEMVs; more through the
-// library's GEMM, a low-bit matrix after one dequantization.
+// rows (out says which); one token through the decode GEMVs; more, a low-bit
+// matrix after one dequantization, through the tile GEMM (partial sums as well)
+// where its ranges of K fill the GPU, else the library's.
 int project_rows(grout_engine* e, const Mat* m, int np, const void* x, uint16_t* y, float* parts,
                  int rows, int k, Proj* out) {
   int n = 0;
-  bool few = true;
+  bool few = true, tile = true;
   for (int i = 0; i < np; ++i) {
     few = few && grout::tok_gemm_ok(m[i].fmt, rows, m[i].rows, k);
+    tile = tile && grout::tile_gemm_ok(rows, m[i].rows, k);
     n += m[i].rows;
   }
+  tile = tile && !few && grout::tile_gemm_pays(rows, n);
   *out = Proj{};
-  if (few) {
-    out->splits = grout::tok_gemm_splits(rows, n, k);
+  if (few || tile) {
+    out->splits = few ? grout::tok_gemm_splits(rows, n, k) : grout::tile_gemm_splits(rows, n, k);
     out->parts = parts;
   }
   if (few && np == 2 && grout::tok_gemm_pair_ok(m[0].fmt, m[1].fmt))
@@ -258,7 +261,12 @@ int project_rows(grout_engine* e, const Mat* m, int np, const void* x, uint16_t*
     } else {
       const void* w = nullptr;
       GROUT_CHECK(mat_f16(e, m[i], k, &w));
-      GROUT_CHECK(gemm_rows(e, w, x, y + col, rows, m[i].rows, k, n));
+      if (tile)
+        GROUT_CHECK(hip_status(grout::launch_tile_gemm(w, x, y + col, parts + col, n, rows,
+                                                       m[i].rows, k, out->splits, e->stream),
+                               "tile_gemm"));
+      else
+        GROUT_CHECK(gemm_rows(e, w, x, y + col, rows, m[i].rows, k, n));
     }
     col += m[i].rows;
   }
@@ -270,8 +278,9 @@ size_t parts_bytes(const grout_engine* e, int cap) {
   const auto& c = e->cfg;
   size_t mx = 0;
   auto see = [&](int n, int k) {
-    for (int r = 2; r <= std::min(cap, grout::kTokMax); ++r) {
-      const int s = grout::tok_gemm_splits(r, n, k);
+    for (int r = 2; r <= std::min(cap, grout::kTileMax); ++r) {
+      const int s = std::max(r <= grout::kTokMax ? grout::tok_gemm_splits(r, n, k) : 1,
+                             grout::tile_gemm_pays(r, n) ? grout::tile_gemm_splits(r, n, k) : 1);
       if (s > 1) mx = std::max(mx, (size_t)s * r * n * sizeof(float));
     }
   };

@@ -154,6 +154,15 @@ hipError_t launch_tok_gemm_pair(int fmt_a, const void* Wa, int Na, int fmt_b, co
                                 int Nb, const void* x, void* y, float* part, long ldy, int M,
                                 int K, int splits, hipStream_t stream);
 
+// Projections of a longer prompt over f16 weights (tile_gemm.hip); arguments
+// as launch_tok_gemm's.
+constexpr int kTileMax = 4096;  // tokens up to which it may be the faster route
+bool tile_gemm_ok(int M, int N, int K);
+bool tile_gemm_pays(int M, int N);
+int tile_gemm_splits(int M, int N, int K);
+hipError_t launch_tile_gemm(const void* W, const void* x, void* y, float* part, long ldy, int M,
+                            int N, int K, int splits, hipStream_t stream);
+
 // Writes the 16x16 C fragment of A x B for A[i][k] = i*32+k (k < 32), B = I
 // padded, one float per (lane, element): used to confirm the MFMA lane layout.
 hipError_t launch_mfma_layout_probe(float* out64x4, hipStream_t stream);
